@@ -151,6 +151,7 @@ struct EigWorkspace {
     DevBuf<double> tau;    // n c128
     DevBuf<double> d, e;   // tridiagonal
     DevBuf<double> ring;   // 2n^2 c128 exchange ring of the reduction
+    DevBuf<double> sub;    // trailing matrix handed to the one-XCD reduction
     DevBuf<double> z;      // n x nband real eigenvectors of T
     // blocked back-transform: the needed columns as c128 (n x nband), the Gram partials,
     // triangular factors and two nb x nband products of the WY blocks, the column list
@@ -258,6 +259,11 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
                   double* eig, Prof* prof = nullptr);
 void heevx_vectors(hipStream_t s, EigWorkspace& ws, GemmWorkspace& gws, int num_cu, int n, int nband,
                    const double* eig, double* vcc, int ldv, const int* need, int nneed, Prof* prof = nullptr);
+// Looks once per device whether workgroups go to its XCDs in turn, which the one-XCD reductions
+// rely on (call with that device current; without it they are not used).
+void eig_probe_xcds(int num_cu);
+// Forgets the finished reductions of a stream that is about to be destroyed (synchronised).
+void eig_forget_stream(hipStream_t s);
 // Sizes ws for every n <= nmax, so heevx_lowest allocates nothing (a growing workspace
 // frees and allocates, and hipFree waits for the device).
 void heevx_reserve(EigWorkspace& ws, int nmax, int nband);

@@ -144,6 +144,7 @@ int apw_ctx_create(apw_ctx** out, int device, void* hip_stream) {
         c->num_cu = prop.multiProcessorCount;
         try {
             (void)apw::gemm_scratch_init(device);   // per device, once: apw_zgemm_noalloc's workspace
+            apw::eig_probe_xcds(c->num_cu);
         } catch (...) {
             if (c->own_stream) (void)hipStreamDestroy(c->stream);
             delete c;
@@ -162,6 +163,7 @@ int apw_ctx_destroy(apw_ctx* ctx) {
             (void)hipStreamSynchronize(ctx->stream);
             ctx->scratch.release();
             ctx->gws.part.release();
+            apw::eig_forget_stream(ctx->stream);
             if (ctx->own_stream) (void)hipStreamDestroy(ctx->stream);
         }
         delete ctx;

@@ -4,11 +4,13 @@
 // hcc to the host and calls LAPACK zheevx every Davidson iteration
 // (rocm/dngvd_op.hip.cu:146-170).  Same algorithm family as zheevx, all on the device:
 //   1. Householder reduction of the lower triangle to a real symmetric tridiagonal T
-//      (zhetrd 'L' form, unblocked) in one kernel: the trailing matrix is partitioned by
-//      columns over workgroups that are all resident at once, one exchange through a ring
-//      per column.  n <= 704: columns in LDS, vectors in registers; up to 2048: columns in
+//      (zhetrd 'L' form, unblocked): the trailing matrix is partitioned by columns over
+//      workgroups that are all resident at once, one exchange through a ring per column.
+//      n <= 512: on one XCD, through its L2, columns in registers; larger matrices start on the
+//      whole device (n <= 704: columns in LDS, vectors in registers; up to 2048: columns in
 //      registers, rows split over the waves of a workgroup; global memory only where neither
-//      fits the GPU (or in one workgroup, for many small concurrent solves);
+//      fits the GPU) and end there.  One workgroup, with the columns in global memory, for many
+//      small concurrent solves that ask for it;
 //   2. bisection with Sturm counts for eigenvalues 0..nband-1 of T (dstebz form);
 //   3. inverse iteration with partial-pivoting tridiagonal LU and Gram-Schmidt inside
 //      clusters of close eigenvalues (dstein form);
@@ -89,9 +91,26 @@ __device__ inline double2 block_sum2(double a, double b, double* red) {
     return make_double2(sa, sb);
 }
 
-__global__ void k_copy_herm(int n, const double2* __restrict__ h, int ldh, double2* __restrict__ a) {
+// Cross-workgroup exchange of the reduction: a ring with one slot per column step,
+// pre-filled with a NaN bit pattern no arithmetic produces.  Producers store each value with
+// device-scope stores (they bypass the non-coherent per-XCD caches); consumers poll the
+// slots they need with device-scope loads until no word holds the pattern.  Every value
+// validates itself, so there is no flag, no fence and no grid barrier: one memory round trip
+// per column.  The check assumes a 16-byte load returns each 8-byte half whole (one
+// request); a torn half could only pass as a wrong value, which k_bisect's finiteness test
+// catches when it is not finite.
+constexpr unsigned long long RING_EMPTY = 0x7ff4dead5eed0001ull;
+
+// What a reduction needs before it starts, in one launch: a = hcc (both triangles from the
+// lower one), nz words of bar zeroed, and the exchange ring filled with its empty pattern.
+__global__ void k_prep(int n, const double2* __restrict__ h, int ldh, double2* __restrict__ a,
+                       unsigned* __restrict__ bar, int nz, double2* __restrict__ ring, size_t nring) {
+    const size_t first = blockIdx.x * (size_t)blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
+    const double empty = __longlong_as_double((long long)RING_EMPTY);
+    if (first < (size_t)nz) bar[first] = 0u;
+    for (size_t i = first; i < nring; i += stride) ring[i] = make_double2(empty, empty);
     const size_t total = (size_t)n * n;
-    for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
+    for (size_t t = first; t < total; t += stride) {
         const int i = (int)(t % n), j = (int)(t / n);
         double2 v;
         if (i > j) {
@@ -104,10 +123,6 @@ __global__ void k_copy_herm(int n, const double2* __restrict__ h, int ldh, doubl
         }
         a[t] = v;
     }
-}
-
-__global__ void k_zero_u32(unsigned* p, int n) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0u;
 }
 
 // Reflector (zlarfg convention) of x[0..mx): P^H x = beta e_1, P = I - tau v v^H, v[0] = 1.
@@ -139,33 +154,19 @@ __device__ void make_reflector(const double2* xs, int mx, double2* vo, double2& 
     __syncthreads();
 }
 
-// Cross-workgroup exchange of the reduction: a ring with one slot per column step,
-// pre-filled with a NaN bit pattern no arithmetic produces.  Producers store each value with
-// device-scope stores (they bypass the non-coherent per-XCD caches); consumers poll the
-// slots they need with device-scope loads until no word holds the pattern.  Every value
-// validates itself, so there is no flag, no fence and no grid barrier: one memory round trip
-// per column.  The check assumes a 16-byte load returns each 8-byte half whole (one
-// request); a torn half could only pass as a wrong value, which k_bisect's finiteness test
-// catches when it is not finite.
-constexpr unsigned long long RING_EMPTY = 0x7ff4dead5eed0001ull;
-
-__global__ void k_fill_ring(double2* ring, size_t count) {
-    const double e = __longlong_as_double((long long)RING_EMPTY);
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x)
-        ring[i] = make_double2(e, e);
-}
-
 // 16-byte forms: one vector buffer load / store per value with the device-scope cache
 // policy (sc1, the bits of the 8-byte device-scope atomics).  Each 8-byte half
 // still validates itself, so a load that sees one half written and the other not simply
 // polls again.  r spans one step's slot (2n values); i is the value's index in it.
 typedef unsigned ring_u4 __attribute__((ext_vector_type(4)));
+typedef unsigned ring_u2 __attribute__((ext_vector_type(2)));
 constexpr int RING_SC1 = 16;
 __device__ inline __amdgpu_buffer_rsrc_t ring_rsrc(const double2* slot, int count) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<double2*>(slot), 0, count * (int)sizeof(double2), 0x00020000);
 }
+template <int POLICY = RING_SC1>
 __device__ inline void ring_put16(__amdgpu_buffer_rsrc_t r, int i, double2 v) {
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ring_u4, v), r, (unsigned)i * 16u, 0, RING_SC1);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ring_u4, v), r, (unsigned)i * 16u, 0, POLICY);
 }
 __device__ inline bool ring_get16(__amdgpu_buffer_rsrc_t r, int i, double2& v) {
     v = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, (unsigned)i * 16u, 0, RING_SC1));
@@ -388,6 +389,319 @@ __device__ inline double2 row_bcast(const double2 (&x)[R], int i) {
         if (r == (i >> 6)) t = x[r];
     return make_double2(lane_bcast(t.x, i & 63), lane_bcast(t.y, i & 63));
 }
+// ---- reductions on one XCD ----------------------------------------------------------------
+// The exchange of the device-wide forms is a store and a load through memory, because the eight
+// XCDs have an L2 each: 1.6 us from 32 workgroups' publications to the last poll, whatever the
+// step computes.  Workgroups of one XCD share its L2: there a store without the device-scope
+// policy and a load that only misses the CU's own cache (sc1) meet, and the same exchange takes
+// 0.66 us (measured, 32 workgroups polling 32 values).  Workgroups go to the XCDs in turn, so a
+// grid of 8 W puts W of them on each; those on the XCD that the launch names do the reduction
+// and the others leave at once.  join (zero before the launch) counts the arrivals there.
+// Returns the workgroup's rank among the W, or -1 (leave).  All of its waves call it.
+constexpr int RING_XCD = 0;    // store policy of the one-XCD form: into the shared L2
+__device__ inline unsigned xcc_id() { return __builtin_amdgcn_s_getreg(((4 - 1) << 11) | 20) & 15u; }   // HW_REG_XCC_ID
+__device__ inline int xcd_join(unsigned* join, int W, unsigned xcc) {
+    __shared__ int rank;
+    if (threadIdx.x == 0) {
+        const int r = xcc_id() == xcc ? (int)atomicAdd(join, 1u) : -1;
+        rank = r < W ? r : -1;
+    }
+    __syncthreads();
+    return rank;
+}
+
+__global__ void k_xcc_ids(unsigned* ids) {
+    if (threadIdx.x == 0) ids[blockIdx.x] = xcc_id();
+}
+
+// Sums over the 64 lanes of 2 NC values at once, NC <= 4: the first stages exchange halves of the
+// values between the two lanes of a pair, so that each stage handles half as many (58
+// instructions for eight values, against 8 x 23 one by one).  The pairs of the stages are the
+// lane involutions that DPP has: l -> 15 - l, 7 - l, 3 - l, l ^ 1 within 16, 8, 4, 2 lanes, then
+// 16 and 32 lanes apart.  Returns value j in the lanes whose bits 3, 2, 1 are bits 0, 1, 2 of j.
+template <int CTRL>
+__device__ inline double pair_merge(double keep0, double keep1, bool hi) {
+    const double keep = hi ? keep1 : keep0, send = hi ? keep0 : keep1;
+    return keep + dppm_d<CTRL>(send);
+}
+__device__ inline double sum_rows_swapped(double v) {   // the same lane of the four 16-lane rows
+    {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+        v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    }
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+template <int NC>
+__device__ inline double wave_sums(const double2 (&p)[NC], int lane) {
+    double a[4], v;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (c < NC) a[c] = pair_merge<0x140>(p[c].x, p[c].y, lane & 8);
+    if constexpr (NC == 1) {
+        v = a[0] + dppm_d<0x141>(a[0]);
+    } else {
+        a[0] = pair_merge<0x141>(a[0], a[1], lane & 4);
+        if constexpr (NC > 2) a[2] = pair_merge<0x141>(a[2], NC > 3 ? a[3] : 0.0, lane & 4);
+        v = a[0];
+    }
+    v = NC > 2 ? pair_merge<0x1B>(a[0], a[2], lane & 2) : v + dppm_d<0x1B>(v);
+    v += dppm_d<0xB1>(v);
+    return sum_rows_swapped(v);
+}
+
+// One-XCD reduction for n <= 64 R (zhetrd 'L' steps as in k_tridiag_reg, another order of work).
+// Every wave of the W workgroups is a unit: unit u owns the columns u, u + U, ... (U = 4 W) in
+// registers and holds all rows of the vectors (lane l: rows l + 64 r).  The four waves of a
+// workgroup poll a quarter of the rows each and pass q, the column and v through LDS.
+// A step is a serial chain -- exchange, sums over lanes, arithmetic -- so what can leave it does:
+//   * the projection is taken on the corrected column w itself, not on the reflector
+//     v = (w - beta e) / (alpha - beta) made from it: units publish q = A^H w, and
+//     p = A^H v = (q - beta (column k+1)) / (alpha - beta), whose second operand the exchange
+//     carries anyway (|alpha - beta| >= |beta|: no cancellation beyond w's own rounding).  The
+//     norm, the square root, the reciprocals and v are formed while q is on its way;
+//   * the coefficients (y_c, v_c) of an own column's update are formed in every lane from row c
+//     of q, the column and v in LDS, not broadcast from the lane that holds row c.
+// Every unit forms the same bits of w, beta and v: the next v follows from this one with a factor
+// |y0 / (alpha - beta)|, so copies that differ in the last place would part at every step.
+template <int R, int NC>
+__global__ __launch_bounds__(NT) void k_tridiag_xcd(const double2* __restrict__ A, int n, int W,
+                                                    double2* __restrict__ V, int ldv, double2* __restrict__ tau,
+                                                    double* __restrict__ d, double* __restrict__ e, double2* ring,
+                                                    unsigned* abort_flag, unsigned* join, unsigned xcc) {
+    constexpr int NW = NT / 64;
+    constexpr unsigned FAR = 0xfffffff0u;   // out of every buffer's range: loads read zero
+    constexpr int RS = (R + NW - 1) / NW;   // row chunks a wave polls
+    __shared__ double2 gq[2][64 * R], gc[2][64 * R], gv[2][64 * R];   // q_k, column k+1, v_k by row
+    const int wg = __builtin_amdgcn_readfirstlane(xcd_join(join, W, xcc));
+    if (wg < 0) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int unit = wg * NW + wave, U = W * NW;
+    if (wg * NW >= n) return;   // no column in the workgroup
+    const __amdgpu_buffer_rsrc_t rs = ring_rsrc(ring, 2 * n * n);
+    // value j of wave_sums in this lane: part j & 1 of own column j >> 1
+    const int pub = ((lane >> 3) & 1) | ((lane >> 1) & 2) | ((lane << 1) & 4);
+    const bool publisher = (lane & 0x31) == 0 && (pub >> 1) < NC;
+    double2 cols[NC][R], v[R], y[R], w[R];
+#pragma unroll
+    for (int lc = 0; lc < NC; ++lc) {
+        const int c = unit + lc * U;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int i = lane + 64 * r;
+            cols[lc][r] = (c < n && i < n) ? A[(size_t)c * n + i] : make_double2(0.0, 0.0);
+        }
+    }
+    double2 t, sc;
+    double beta, c2 = 0.0;
+    auto to_y = [&](double2 p, double2 vv) {
+        const double2 tp = cmul(t, p);
+        return make_double2(fma(-c2, vv.x, tp.x), fma(-c2, vv.y, tp.y));
+    };
+    auto to_p = [&](double2 q, double2 c) {
+        return cmul(sc, make_double2(fma(-beta, c.x, q.x), fma(-beta, c.y, q.y)));
+    };
+    // Publishes q_{k+1} of the own columns c > k + 1 (and column k + 2 by its owner) into slot
+    // k + 1; for k >= 0 after the rank-2 update of step k.  w is zero on rows <= k + 1 and past n;
+    // v and y on rows <= k and past n (row k + 1 of a column changes and is not read again).
+    auto update_and_project = [&](int k, bool update, const double2* q, const double2* col, const double2* vl) {
+        const int s = (k + 1) * 2 * n;
+        const int r0 = (k + 2) >> 6;   // rows below 64 r0 are done with
+        double2 p[NC];
+#pragma unroll
+        for (int lc = 0; lc < NC; ++lc) {
+            const int c = unit + lc * U;
+            p[lc] = make_double2(0.0, 0.0);
+            if (c > k + 1 && c < n) {   // uniform over the wave
+                double2 yc = make_double2(0.0, 0.0), vc = yc;
+                if (update) {
+                    vc = vl[c];
+                    yc = to_y(to_p(q[c], col[c]), vc);
+                }
+                double pr = 0, pi = 0;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    if (r < r0) continue;
+                    double2 a = cols[lc][r];
+                    if (update) {
+                        a.x = fma(-yc.x, v[r].x, a.x);
+                        a.x = fma(-yc.y, v[r].y, a.x);
+                        a.x = fma(-vc.x, y[r].x, a.x);
+                        a.x = fma(-vc.y, y[r].y, a.x);
+                        a.y = fma(-yc.x, v[r].y, a.y);
+                        a.y = fma(yc.y, v[r].x, a.y);
+                        a.y = fma(-vc.x, y[r].y, a.y);
+                        a.y = fma(vc.y, y[r].x, a.y);
+                        cols[lc][r] = a;
+                    }
+                    pr = fma(a.x, w[r].x, pr);
+                    pr = fma(a.y, w[r].y, pr);
+                    pi = fma(a.x, w[r].y, pi);
+                    pi = fma(-a.y, w[r].x, pi);
+                }
+                p[lc] = make_double2(pr, pi);
+                if (c == k + 2) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const int i = lane + 64 * r;
+                        if (i >= k + 2 && i < n) ring_put16<RING_XCD>(rs, s + n + i, cols[lc][r]);
+                    }
+                }
+            }
+        }
+        const double sum = wave_sums<NC>(p, lane);
+        const int c = unit + (pub >> 1) * U;
+        if (publisher && c > k + 1 && c < n)
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(ring_u2, sum), rs,
+                                                  (unsigned)(s + c) * 16u + 8u * (pub & 1), 0, RING_XCD);
+    };
+    // Reflector of w (rows > k0; alpha at row k0 + 1): v, tau, beta, sc = 1 / (alpha - beta).
+    // Off the chain: q is in flight.
+    auto reflector = [&](int k0, double2 alpha, double dk) {
+        const int r0 = (k0 + 1) >> 6;
+        double s2 = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (r < r0) continue;
+            const int i = lane + 64 * r;
+            if (i > k0 + 1) s2 += w[r].x * w[r].x + w[r].y * w[r].y;   // zero past n
+        }
+        const double xn2 = wave_sum(s2);
+        if (xn2 == 0.0 && alpha.y == 0.0) {
+            t = make_double2(0.0, 0.0);
+            beta = alpha.x;
+            sc = make_double2(0.0, 0.0);
+        } else {
+            const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xn2);
+            beta = alpha.x >= 0 ? -nrm : nrm;
+            const double rb = 1.0 / beta;
+            t = make_double2((beta - alpha.x) * rb, -alpha.y * rb);
+            const double2 den = make_double2(alpha.x - beta, alpha.y);
+            const double rd = 1.0 / (den.x * den.x + den.y * den.y);
+            sc = make_double2(den.x * rd, -den.y * rd);
+        }
+        double2* vl = gv[k0 & 1];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (r < r0) continue;
+            const int i = lane + 64 * r;
+            v[r] = (i == k0 + 1) ? make_double2(1.0, 0.0) : cmul(w[r], sc);   // w: zero on rows <= k0, past n
+            if (r % NW == wave) {
+                vl[i] = v[r];
+                if (wg == 0 && i > k0 && i < n) V[(size_t)k0 * ldv + i] = v[r];
+            }
+        }
+        if (unit == 0 && lane == 0) {
+            tau[k0] = t;
+            d[k0] = dk;
+            e[k0] = beta;
+        }
+    };
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = lane + 64 * r;
+        w[r] = (i >= 1 && i < n) ? A[i] : make_double2(0.0, 0.0);
+        y[r] = v[r] = make_double2(0.0, 0.0);
+    }
+    update_and_project(-1, false, nullptr, nullptr, nullptr);
+    reflector(0, A[1], A[0].x);
+    for (int k = 0; k < n - 1; ++k) {
+        const int r0 = (k + 1) >> 6;
+        double2 *q = gq[k & 1], *col = gc[k & 1];
+        const double2* vl = gv[k & 1];
+        // ---- own share of q_k and column k+1 (rows > k) into LDS ----
+        {
+            double2 pq[RS], pw[RS];
+            unsigned oq[RS], oc[RS], spins = 0;
+#pragma unroll
+            for (int j = 0; j < RS; ++j) {
+                const int i = lane + 64 * (wave + NW * j);
+                const bool in = i > k && i < n;
+                oq[j] = in ? (unsigned)(k * 2 * n + i) * 16u : FAR;
+                oc[j] = in ? (unsigned)(k * 2 * n + n + i) * 16u : FAR;
+            }
+            // the offset is opaque to the compiler at every poll: with nothing in the loop that
+            // it takes for a write to the ring, it hoisted the loads and polled registers
+            auto load = [&](unsigned& off) {
+                asm volatile("" : "+v"(off));
+                return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, RING_SC1));
+            };
+            auto full = [](double2 x) {
+                return (unsigned long long)__double_as_longlong(x.x) != RING_EMPTY &&
+                       (unsigned long long)__double_as_longlong(x.y) != RING_EMPTY;
+            };
+            while (true) {
+                bool ok = true;
+#pragma unroll
+                for (int j = 0; j < RS; ++j) {
+                    pq[j] = load(oq[j]);
+                    pw[j] = load(oc[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < RS; ++j) ok = ok && full(pq[j]) && full(pw[j]);
+                if (__all(ok)) break;
+                // every wave leaves: its values arrive, it sees the abort word, or it raises it
+                if ((++spins & 31u) == 0) {
+                    int st = 0;
+                    if (lane == 0) {
+                        st = __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+                        if (!st && spins > SPIN_LIMIT) {
+                            atomicExch(abort_flag, 1u);
+                            st = 1;
+                        }
+                    }
+                    if (__shfl(st, 0, 64)) break;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < RS; ++j) {
+                const int i = lane + 64 * (wave + NW * j);
+                if (i < 64 * R) {
+                    q[i] = pq[j];
+                    col[i] = pw[j];
+                }
+            }
+            __syncthreads();
+        }
+        // ---- p = sc (q - beta column), mu = v^H p, y = tau p - (|tau|^2 mu / 2) v ----
+        double mr = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (r < r0) continue;
+            w[r] = col[lane + 64 * r];
+            y[r] = to_p(q[lane + 64 * r], w[r]);
+            mr = fma(v[r].x, y[r].x, mr);
+            mr = fma(v[r].y, y[r].y, mr);
+        }
+        const double mu = wave_sum(mr);
+        c2 = 0.5 * (t.x * t.x + t.y * t.y) * mu;
+        const double2 y0 = to_y(to_p(q[k + 1], col[k + 1]), make_double2(1.0, 0.0));   // v_k[k+1] = 1
+        const double dk1 = col[k + 1].x - 2.0 * y0.x;
+        // ---- y, and w = column k+1 after the rank-2 update (rows > k+1) ----
+        auto corrected = [&](double2 c, double2 vi, double2 yi) {   // c - v conj(y0) - y
+            const double2 a1 = cconjmul(y0, vi);
+            return make_double2(c.x - (a1.x + yi.x), c.y - (a1.y + yi.y));
+        };
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (r < r0) continue;
+            y[r] = to_y(y[r], v[r]);
+            w[r] = lane + 64 * r > k + 1 ? corrected(w[r], v[r], y[r]) : make_double2(0.0, 0.0);
+        }
+        if (k < n - 2) {
+            const double2 v1 = vl[k + 2];
+            const double2 alpha = corrected(col[k + 2], v1, to_y(to_p(q[k + 2], col[k + 2]), v1));
+            update_and_project(k, true, q, col, vl);
+            reflector(k + 1, alpha, dk1);
+        } else if (unit == 0 && lane == 0) {
+            d[k + 1] = dk1;
+        }
+    }
+}
+
 // Householder tridiagonalisation (lower), LDS-resident columns, vectors in registers.
 // Same ownership and exchange as k_tridiag_fused; what changes is where the per-column work
 // happens.  Every wave holds the full vectors v_k, y_k and the next reflector v_{k+1} in
@@ -395,11 +709,15 @@ __device__ inline double2 row_bcast(const double2 (&x)[R], int i) {
 // reflector are formed with wave reductions only, and one pass over each own column both
 // applies the rank-2 update of step k and accumulates p_{k+1} = A_{k+1}^H v_{k+1} (the
 // column is read and written once per step).  Workgroup barriers: the gather's only.
+// kstop > 0: the reduction stops before the reflector of column kstop and leaves the trailing
+// matrix A_kstop (rows and columns kstop .. n-1; row kstop only in its first column) in sub,
+// leading dimension n - kstop, for the one-XCD form.
 template <int R, int NTR>
 __global__ __launch_bounds__(NTR) void k_tridiag_reg(const double2* __restrict__ A, int n, int ncol,
                                                     double2* __restrict__ V, double2* __restrict__ tau,
                                                     double* __restrict__ d, double* __restrict__ e,
-                                                    double2* __restrict__ ring, unsigned* abort_flag) {
+                                                    double2* __restrict__ ring, unsigned* abort_flag,
+                                                    int kstop, double2* __restrict__ sub) {
     extern __shared__ __align__(16) unsigned char smem[];
     double2* Al = reinterpret_cast<double2*>(smem);   // Al[lc * n + i] = A[i][c], c = blockIdx.x + lc * nwg
     double2* gs = Al + (size_t)ncol * n;                // gathered p and column, two buffers of 2n
@@ -592,6 +910,7 @@ __global__ __launch_bounds__(NTR) void k_tridiag_reg(const double2* __restrict__
                 w[r].y -= a1.y + a2.y;
             }
         }
+        if (k + 1 == kstop) break;   // column k+1 is in w, columns c > k+1 lack step k's update
         const double dk1 = row_bcast<R>(w, k + 1).x;
         if (m >= 2) {
             double2 tn;
@@ -617,6 +936,39 @@ __global__ __launch_bounds__(NTR) void k_tridiag_reg(const double2* __restrict__
             d[k + 1] = dk1;
         }
     }
+    if (kstop > 0) {
+        // hand the trailing matrix over: column kstop is in w; own columns after it take the
+        // last rank-2 update on their way out
+        const int lds = n - kstop;
+        if (bid == 0 && wave == 0) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int i = lane + 64 * r;
+                if (i >= kstop && i < n) sub[i - kstop] = w[r];
+            }
+        }
+        for (int lc = (kstop + 1 - bid + nwg - 1) / nwg + wave; lc < ncol; lc += NW) {
+            const int c = bid + lc * nwg;
+            if (c >= n) break;
+            const double2 yc = row_bcast<R>(y, c), vc = row_bcast<R>(v, c);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int i = lane + 64 * r;
+                if (i > kstop && i < n) {
+                    double2 a = Al[(size_t)lc * n + i];
+                    a.x = fma(-yc.x, v[r].x, a.x);
+                    a.x = fma(-yc.y, v[r].y, a.x);
+                    a.x = fma(-vc.x, y[r].x, a.x);
+                    a.x = fma(-vc.y, y[r].y, a.x);
+                    a.y = fma(-yc.x, v[r].y, a.y);
+                    a.y = fma(yc.y, v[r].x, a.y);
+                    a.y = fma(-vc.x, y[r].y, a.y);
+                    a.y = fma(vc.y, y[r].x, a.y);
+                    sub[(size_t)(c - kstop) * lds + (i - kstop)] = a;
+                }
+            }
+        }
+    }
 }
 
 // Householder tridiagonalisation (lower) for large n (up to 64 * NW * CH rows): the own
@@ -633,7 +985,8 @@ template <int CH, int NC, int NW>
 __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restrict__ A, int n, int ncol,
                                                          double2* __restrict__ V, double2* __restrict__ tau,
                                                          double* __restrict__ d, double* __restrict__ e,
-                                                         double2* __restrict__ ring, unsigned* abort_flag) {
+                                                         double2* __restrict__ ring, unsigned* abort_flag,
+                                                         int kstop, double2* __restrict__ sub) {
     extern __shared__ __align__(16) unsigned char smem[];
     double2* yl = reinterpret_cast<double2*>(smem);   // y_k by row
     double2* vl = yl + n;                              // v_k by row
@@ -894,6 +1247,7 @@ __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restr
                     vl[i] = v[ch];
                 }
             }
+            if (k + 1 == kstop) break;   // y_k, v_k in yl, vl; column k+1 in w
             double2 tn;
             double bn;
             reflector(k + 1, tn, bn);
@@ -915,6 +1269,34 @@ __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restr
             t = tn;
         } else if (bid == 0 && threadIdx.x == 0) {
             d[k + 1] = dk1;
+        }
+    }
+    if (kstop > 0) {   // hand the trailing matrix over, as in k_tridiag_reg
+        const int lds = n - kstop;
+        __syncthreads();
+#pragma unroll
+        for (int ch = 0; ch < CH; ++ch) {
+            const int i = 64 * (wave + NW * ch) + lane;
+            if (i < kstop || i >= n) continue;
+            if (bid == 0) sub[i - kstop] = w[ch];
+            if (i == kstop) continue;
+#pragma unroll
+            for (int lc = 0; lc < NC; ++lc) {
+                const int c = bid + lc * nwg;
+                if (lc < ncol && c > kstop && c < n) {
+                    const double2 yc = yl[c], vc = vl[c], vi = vl[i], yi = yl[i];
+                    double2 a = cols[lc][ch];
+                    a.x = fma(-yc.x, vi.x, a.x);
+                    a.x = fma(-yc.y, vi.y, a.x);
+                    a.x = fma(-vc.x, yi.x, a.x);
+                    a.x = fma(-vc.y, yi.y, a.x);
+                    a.y = fma(-yc.x, vi.y, a.y);
+                    a.y = fma(yc.y, vi.x, a.y);
+                    a.y = fma(-vc.x, yi.y, a.y);
+                    a.y = fma(vc.y, yi.x, a.y);
+                    sub[(size_t)(c - kstop) * lds + (i - kstop)] = a;
+                }
+            }
         }
     }
 }
@@ -1665,52 +2047,136 @@ __global__ __launch_bounds__(1024) void k_chol_inv(int n, const double2* __restr
 
 }  // namespace
 
-// Launches of the multi-workgroup reduction, whose workgroups wait on each other's ring
-// values, may run at the same time on several streams only while all their workgroups fit
-// on the GPU together (each workgroup fits one CU): then none can wait on a workgroup that
-// cannot start, and ordinary kernels beside them always finish and free their CUs.  A
-// device-wide ledger keeps the reductions not known to have finished (launch order, width);
-// a new one whose width would take the running total past the CU count first makes its
-// stream wait for the oldest of them, as many as needed.  Every set of reductions that can
-// run together then has at most num_cu workgroups: a later one overlaps an earlier one only
-// if it did not wait for it, and then the earlier one was counted against its width.
+// Launches of the multi-workgroup reductions, whose workgroups wait on each other's ring values,
+// may run at the same time on several streams only while all their workgroups fit on the GPU
+// together (each workgroup fits one CU): then none can wait on a workgroup that cannot start, and
+// ordinary kernels beside them always finish and free their CUs.  A device-wide ledger keeps the
+// reductions not known to have finished, in launch order, with the CUs they need on each XCD: a
+// device-wide form an eighth of its workgroups on every XCD, a one-XCD form all of its workgroups
+// on one, the least loaded.  A new one that would not fit first makes its stream wait for the
+// oldest of the other streams' (its own stream's are over before it starts), as many as needed.
+// Every set of reductions that can run together then fits: a later one overlaps an earlier one
+// only if it did not wait for it, and then the earlier one was counted.
 namespace {
+constexpr int NXCD = 8;
+struct SpinEntry {
+    hipEvent_t ev;     // completion
+    hipStream_t s;
+    int w, xcd;        // workgroups; the XCD they run on, or -1: all
+};
 struct SpinLedger {
     std::mutex m;
-    std::deque<std::pair<hipEvent_t, int>> live;   // (completion event, workgroups)
-    std::vector<hipEvent_t> pool;
+    std::deque<SpinEntry> live;
+    std::vector<SpinEntry> pool;   // finished
+    // one-XCD forms: the XCC ids in the order in which workgroups go to them, once probed
+    bool probed = false, xcd_ok = false;
+    unsigned xcc[NXCD] = {};
 };
 SpinLedger g_ledger[64];
 
-void spin_launch(const void* fn, dim3 grid, dim3 block, void** args, unsigned lds, hipStream_t s, int num_cu) {
+SpinLedger& ledger() {
     int dev = 0;
     APW_HIP(hipGetDevice(&dev));
-    SpinLedger& L = g_ledger[dev & 63];
+    return g_ledger[dev & 63];
+}
+
+// xcd: choose an XCD and pass its XCC id in *xcc (an argument of the kernel).
+void spin_launch(const void* fn, dim3 grid, dim3 block, void** args, unsigned lds, hipStream_t s, int num_cu,
+                 bool xcd = false, unsigned* xcc = nullptr) {
+    SpinLedger& L = ledger();
     std::lock_guard<std::mutex> lock(L.m);
-    const int w = (int)grid.x;
-    APW_CHECK(w <= num_cu, "tridiagonal reduction: %d workgroups on %d CUs", w, num_cu);
-    while (!L.live.empty() && hipEventQuery(L.live.front().first) == hipSuccess) {
-        L.pool.push_back(L.live.front().first);
+    const int w = xcd ? (int)grid.x / NXCD : (int)grid.x;
+    APW_CHECK(w <= (xcd ? num_cu / NXCD : num_cu), "tridiagonal reduction: %d workgroups on %d CUs", w, num_cu);
+    while (!L.live.empty() && hipEventQuery(L.live.front().ev) == hipSuccess) {
+        L.pool.push_back(L.live.front());
         L.live.pop_front();
     }
-    int used = 0;
-    for (const auto& g : L.live) used += g.second;
-    for (auto it = L.live.begin(); used + w > num_cu && it != L.live.end(); ++it) {
-        APW_HIP(hipStreamWaitEvent(s, it->first, 0));
-        used -= it->second;
+    // load[x]: eighths of CUs, a device-wide width rounded up to the same share of every XCD
+    int load[NXCD] = {};
+    auto add = [&](const SpinEntry& g, int sign) {
+        for (int x = 0; x < NXCD; ++x)
+            if (g.xcd < 0 || g.xcd == x) load[x] += sign * (g.xcd < 0 ? (g.w + NXCD - 1) / NXCD * NXCD : NXCD * g.w);
+    };
+    for (const auto& g : L.live)
+        if (g.s != s) add(g, 1);
+    auto place = [&]() {   // the XCD to run on (0 for a device-wide form), -1 if it does not fit yet
+        if (xcd) {
+            const int x = (int)(std::min_element(load, load + NXCD) - load);
+            return load[x] + NXCD * w <= num_cu ? x : -1;
+        }
+        return *std::max_element(load, load + NXCD) + (w + NXCD - 1) / NXCD * NXCD <= num_cu ? 0 : -1;
+    };
+    int at = place();
+    for (auto it = L.live.begin(); at < 0 && it != L.live.end(); ++it) {
+        if (it->s == s) continue;
+        APW_HIP(hipStreamWaitEvent(s, it->ev, 0));
+        add(*it, -1);
+        at = place();
     }
+    if (xcd) *xcc = L.xcc[at];
     APW_HIP(hipLaunchKernel(fn, grid, block, args, lds, s));
     hipEvent_t ev;
     if (!L.pool.empty()) {
-        ev = L.pool.back();
+        ev = L.pool.back().ev;
         L.pool.pop_back();
     } else {
         APW_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     }
     APW_HIP(hipEventRecord(ev, s));
-    L.live.emplace_back(ev, w);
+    L.live.push_back(SpinEntry{ev, s, w, xcd ? at : -1});
+}
+
+bool xcd_available() {
+    SpinLedger& L = ledger();
+    std::lock_guard<std::mutex> lock(L.m);
+    return L.xcd_ok;
 }
 }  // namespace
+
+// An event may outlive the stream it was last recorded on, but not be queried then: a query that
+// looked at a freed stream has failed as if that stream were being captured.
+void eig_forget_stream(hipStream_t s) {
+    SpinLedger& L = ledger();
+    std::lock_guard<std::mutex> lock(L.m);
+    auto drop = [&](auto& list) {
+        for (auto it = list.begin(); it != list.end();) {
+            if (it->s == s) {
+                (void)hipEventDestroy(it->ev);
+                it = list.erase(it);
+            } else {
+                ++it;
+            }
+        }
+    };
+    drop(L.live);
+    drop(L.pool);
+}
+
+void eig_probe_xcds(int num_cu) {
+    SpinLedger& L = ledger();
+    std::lock_guard<std::mutex> lock(L.m);
+    if (L.probed) return;
+    L.probed = true;
+    if (num_cu != 256) return;   // 8 XCDs of 32 CUs; a partition of the GPU keeps the device-wide forms
+    constexpr int nb = 256;
+    unsigned ids[nb];
+    DevBuf<unsigned> dev;
+    dev.reserve(nb);
+    hipStream_t s;
+    APW_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+    hipLaunchKernelGGL(k_xcc_ids, dim3(nb), dim3(64), 0, s, dev.get());
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(ids, dev.get(), sizeof(ids), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    (void)hipStreamDestroy(s);
+    APW_HIP(e);
+    bool ok = true;
+    for (int b = 0; b < nb; ++b) ok = ok && ids[b] == ids[b % NXCD];
+    for (int x = 0; x < NXCD; ++x)
+        for (int z = 0; z < x; ++z) ok = ok && ids[x] != ids[z];
+    std::copy(ids, ids + NXCD, L.xcc);
+    L.xcd_ok = ok;
+}
 
 // sizes of the blocked back-transform's work arrays (doubles) for n x mc
 struct WySizes {
@@ -1774,6 +2240,9 @@ void backtransform_wy(hipStream_t s, EigWorkspace& ws, GemmWorkspace& gws, int n
     APW_LAUNCH_CHECK();
 }
 
+constexpr int XCD_MAX = 512;    // columns the one-XCD form takes: 4 a wave, 8 rows of each a lane
+constexpr int BAR_WORDS = 65;   // [1]: abort word, [64]: xcd_join's count
+
 void heevx_reserve(EigWorkspace& ws, int nmax, int nband) {
     const size_t n = (size_t)std::max(nmax, 1);
     ws.a.reserve(2 * n * n);
@@ -1782,8 +2251,9 @@ void heevx_reserve(EigWorkspace& ws, int nmax, int nband) {
     ws.d.reserve(n);
     ws.e.reserve(n);
     ws.z.reserve(n * (size_t)std::max(nband, 1));
-    ws.bar.reserve(64 + 256);
-    ws.ring.reserve(2 * (2 * n * n));   // the larger of the two exchange rings below
+    ws.bar.reserve(BAR_WORDS);
+    ws.ring.reserve(2 * (2 * n * n));   // the largest of the exchange rings below
+    if ((int)n > XCD_MAX) ws.sub.reserve((size_t)2 * XCD_MAX * XCD_MAX);
     if ((int)n >= WY_MIN_N) wy_reserve(ws, (int)n, std::max(nband, 1));
 }
 
@@ -1792,6 +2262,33 @@ void heevx_lowest(hipStream_t s, EigWorkspace& ws, GemmWorkspace& gws, int num_c
     APW_CHECK(ldv >= n, "heevx: ldv=%d below n=%d", ldv, n);
     heevx_values(s, ws, num_cu, n, ldh, hcc, nband, eig, prof);
     heevx_vectors(s, ws, gws, num_cu, n, nband, eig, vcc, ldv, nullptr, nband, prof);
+}
+
+// The one-XCD reduction of an m x m matrix (both triangles, ld m) into V (ld ldv), tau, d, e;
+// m <= XCD_MAX.  join is zero and the ring empty (2 m^2 values).  NC columns a wave, as few as
+// 32 workgroups of four waves allow, and then no more workgroups than that needs: 18 of them at
+// m = 144 (two columns a wave) take 249 us, 32 take 246; 12 at m = 48 (one column) 69 us, 6 take 74.
+void tridiag_xcd(hipStream_t s, int num_cu, const double2* A, int m, double2* V, int ldv, double2* tau, double* d,
+                 double* e, double2* ring, unsigned* abortp, unsigned* join) {
+    constexpr int NW = NT / 64;
+    const int R = (m + 63) / 64, wmax = num_cu / NXCD;
+    const int nc = (m + NW * wmax - 1) / (NW * wmax);
+    int W = (m + NW * nc - 1) / (NW * nc);
+    const void* fn = nullptr;
+    switch (R) {
+        case 1: fn = reinterpret_cast<const void*>(k_tridiag_xcd<1, 1>); break;
+        case 2: fn = reinterpret_cast<const void*>(k_tridiag_xcd<2, 1>); break;
+        case 3: fn = reinterpret_cast<const void*>(k_tridiag_xcd<3, 2>); break;
+        case 4: fn = reinterpret_cast<const void*>(k_tridiag_xcd<4, 2>); break;
+        case 5: fn = reinterpret_cast<const void*>(k_tridiag_xcd<5, 3>); break;
+        case 6: fn = reinterpret_cast<const void*>(k_tridiag_xcd<6, 3>); break;
+        case 7: fn = reinterpret_cast<const void*>(k_tridiag_xcd<7, 4>); break;
+        default: fn = reinterpret_cast<const void*>(k_tridiag_xcd<8, 4>); break;
+    }
+    APW_CHECK(m <= XCD_MAX && nc <= (R + 1) / 2, "heevx: one-XCD form cannot take m=%d on %d CUs", m, wmax);
+    unsigned xcc = 0;
+    void* args[] = {&A, &m, &W, &V, &ldv, &tau, &d, &e, &ring, &abortp, &join, &xcc};
+    spin_launch(fn, dim3(NXCD * W), dim3(NT), args, 0, s, num_cu, true, &xcc);
 }
 
 void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, const double* hcc, int nband,
@@ -1804,58 +2301,63 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
     ws.d.reserve(n);
     ws.e.reserve(n);
     ws.z.reserve((size_t)n * nband);
-    ws.bar.reserve(64 + 256);
+    ws.bar.reserve(BAR_WORDS);
     double2* A = reinterpret_cast<double2*>(ws.a.get());
-    hipLaunchKernelGGL(k_copy_herm, dim3(std::min(4096, (n * n + 255) / 256)), dim3(256), 0, s, n,
-                       reinterpret_cast<const double2*>(hcc), ldh, A);
+    const int R = (n + 63) / 64;
+    // one XCD takes the reduction up to XCD_MAX columns, where the registers of its 32 CUs hold
+    // them; a larger matrix starts on the whole device and its last XCD_MAX columns are reduced on
+    // one XCD (kstop: the first of them).  n = 512: 2.32 ms on the whole device, 1.53 ms on one
+    // XCD; n = 640: 3.23 ms, 2.27 ms with the last 512 columns there (2.36 with 384, 2.52 with 256)
+    const bool xcd = n > ws.single_max && xcd_available();
+    int kstop = xcd && n > XCD_MAX ? n - XCD_MAX : 0;
+    const bool only_xcd = xcd && kstop == 0;
+    const int ns = n - kstop;   // columns of the one-XCD part
+    const size_t nring_dev = only_xcd ? 0 : (size_t)2 * n * (xcd ? kstop : n);
+    const size_t nring = nring_dev + (xcd ? (size_t)2 * ns * ns : 0);
+    ws.ring.reserve(2 * nring);
+    double2* ring = reinterpret_cast<double2*>(ws.ring.get());
+    if (kstop) ws.sub.reserve((size_t)2 * ns * ns);
+    double2* sub = reinterpret_cast<double2*>(ws.sub.get());
+    const size_t prep_n = std::max((size_t)n * n, nring);
+    hipLaunchKernelGGL(k_prep, dim3((unsigned)std::min<size_t>(2048, (prep_n + 255) / 256)), dim3(256), 0, s, n,
+                       reinterpret_cast<const double2*>(hcc), ldh, A, ws.bar.get(), BAR_WORDS, ring, nring);
     APW_LAUNCH_CHECK();
     if (n > 1) {
-        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, s, ws.bar.get(), 64 + 256);
-        APW_LAUNCH_CHECK();
         // bar[1]: abort word of the exchange polls; V: n x n reflectors
-        APW_CHECK(ws.bar.n >= 2 && ws.v.n >= (size_t)2 * n * n, "heevx: workspace too small for n=%d", n);
+        APW_CHECK(ws.bar.n >= BAR_WORDS && ws.v.n >= (size_t)2 * n * n, "heevx: workspace too small for n=%d", n);
         double2* Vp = reinterpret_cast<double2*>(ws.v.get());
         double2* taup = reinterpret_cast<double2*>(ws.tau.get());
         double* dp = ws.d.get();
         double* ep = ws.e.get();
-        unsigned* barp = ws.bar.get();
+        unsigned* abortp = ws.bar.get() + 1;
+        unsigned* joinp = ws.bar.get() + 64;
+        const double2* Ac = A;
+        // a tuner's trial starts from an empty ring, and leaves one and a clear abort word
+        auto refill = [&] {
+            hipLaunchKernelGGL(k_prep, dim3((unsigned)std::min<size_t>(2048, (prep_n + 255) / 256)), dim3(256), 0, s, n,
+                               reinterpret_cast<const double2*>(hcc), ldh, A, ws.bar.get(), BAR_WORDS, ring, nring);
+            APW_LAUNCH_CHECK();
+        };
         // algorithmic HBM bytes: the matrix read once (16 n^2) and the reflectors written
         // (8 n^2); the per-column hemv and rank-2 update work on LDS-resident columns
         ProfScope ps(prof, s, "eig_tridiag", 24.0 * n * (double)n, 16.0 / 3.0 * n * (double)n * n);
-        // LDS-resident form: the fewest workgroups whose column share fits the LDS budget
         // fused form: v_k, v_{k+1}, y and the gathered column (n each) + scratch, and the
         // own columns when they live in LDS
         const size_t fixed = (size_t)4 * n * sizeof(double2) + 64 * sizeof(double);
-        int nwg = -1, ncol = 0;
-        for (int w = std::max(1, std::min(n / 8, 16)); w <= std::min(num_cu, 256); ++w) {
-            const int nc = (n + w - 1) / w;
-            if (fixed + (size_t)nc * n * sizeof(double2) <= TRIDIAG_LDS_BYTES) {
-                nwg = w;
-                ncol = nc;
-                break;
-            }
-        }
-        const int R = (n + 63) / 64;
         // the row-split register form from n = 705 (measured faster than the LDS-column register
         // form there: 4.3 vs 4.5 ms at n = 768, 6.2 vs 8.0 ms at n = 1024) when n / 8
         // workgroups fit on the GPU; the LDS-column form below that, or to n = 1024 otherwise
         const bool rows_fit = n <= 2048 && (n + 7) / 8 <= std::min(num_cu, 256);
-        if (n <= ws.single_max) {
+        if (only_xcd) {
+            // below
+        } else if (n <= ws.single_max) {
             // one workgroup owns every column (kept in the copy A) and exchanges with itself:
             // an ordinary launch, not ordered against other streams' reductions, so many small
             // solves (batched k-points or cells) reduce at the same time
-            const int ncol1 = n;
-            const size_t lds = fixed;
-            const size_t nring = (size_t)2 * n * (n - 1);
-            ws.ring.reserve(2 * nring);
-            double2* ring = reinterpret_cast<double2*>(ws.ring.get());
-            hipLaunchKernelGGL(k_fill_ring, dim3((unsigned)std::min<size_t>(1024, (nring + 255) / 256)), dim3(256), 0, s,
-                               ring, nring);
-            APW_LAUNCH_CHECK();
             APW_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tridiag_fused<true>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(k_tridiag_fused<true>, dim3(1), dim3(NT), lds, s, A, n, ncol1, Vp, taup, dp, ep, ring,
-                               barp + 1);
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)fixed));
+            hipLaunchKernelGGL(k_tridiag_fused<true>, dim3(1), dim3(NT), fixed, s, A, n, n, Vp, taup, dp, ep, ring,
+                               abortp);
             APW_LAUNCH_CHECK();
         } else if (R <= 11 || (R <= 16 && !rows_fit)) {
             // register form: LDS = own columns + two gather buffers of 2n
@@ -1872,37 +2374,29 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
             // participants up to ~160 of them (measured n = 160..640: 5-17 % faster than the
             // LDS minimum; 192 and 256 workgroups lost again at n = 640)
             w = std::max(w, std::min(std::min(num_cu, 160), n / 4));
-            const size_t nring = (size_t)2 * n * n;
-            ws.ring.reserve(2 * nring);
-            double2* ring = reinterpret_cast<double2*>(ws.ring.get());
             const void* fn = nullptr;
             // threads per workgroup: 512 for 6 <= R <= 12 (measured faster at n = 480, 640: each
             // wave updates fewer columns); 256 otherwise (small n: the extra waves cost more in
             // barriers than they save; R = 16: the register budget of v, y, w, 6 R doubles a lane)
             int ntr = 256;
             switch (R <= 6 ? R : (R <= 8 ? 8 : (R <= 10 ? 10 : (R <= 12 ? 12 : 16)))) {
-                case 1: fn = reinterpret_cast<const void*>(k_tridiag_reg<1, 256>); ntr = 256; break;
-                case 2: fn = reinterpret_cast<const void*>(k_tridiag_reg<2, 256>); ntr = 256; break;
-                case 3: fn = reinterpret_cast<const void*>(k_tridiag_reg<3, 256>); ntr = 256; break;
-                case 4: fn = reinterpret_cast<const void*>(k_tridiag_reg<4, 256>); ntr = 256; break;
-                case 5: fn = reinterpret_cast<const void*>(k_tridiag_reg<5, 256>); ntr = 256; break;
+                case 1: fn = reinterpret_cast<const void*>(k_tridiag_reg<1, 256>); break;
+                case 2: fn = reinterpret_cast<const void*>(k_tridiag_reg<2, 256>); break;
+                case 3: fn = reinterpret_cast<const void*>(k_tridiag_reg<3, 256>); break;
+                case 4: fn = reinterpret_cast<const void*>(k_tridiag_reg<4, 256>); break;
+                case 5: fn = reinterpret_cast<const void*>(k_tridiag_reg<5, 256>); break;
                 case 6: fn = reinterpret_cast<const void*>(k_tridiag_reg<6, 512>); ntr = 512; break;
                 case 8: fn = reinterpret_cast<const void*>(k_tridiag_reg<8, 512>); ntr = 512; break;
                 case 10: fn = reinterpret_cast<const void*>(k_tridiag_reg<10, 512>); ntr = 512; break;
                 case 12: fn = reinterpret_cast<const void*>(k_tridiag_reg<12, 512>); ntr = 512; break;
-                default: fn = reinterpret_cast<const void*>(k_tridiag_reg<16, 256>); ntr = 256; break;
+                default: fn = reinterpret_cast<const void*>(k_tridiag_reg<16, 256>); break;
             }
             // one reduction with wg workgroups (A is only read: it can run again)
             auto run_reg = [&](int wg) {
                 int ncol_r = (n + wg - 1) / wg;
                 const size_t lds = fixed_r + (size_t)ncol_r * n * sizeof(double2);
-                hipLaunchKernelGGL(k_fill_ring, dim3((unsigned)std::min<size_t>(1024, (nring + 255) / 256)), dim3(256),
-                                   0, s, ring, nring);
-                APW_LAUNCH_CHECK();
                 APW_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                const double2* Ac = A;
-                unsigned* abortp = barp + 1;
-                void* args[] = {&Ac, &n, &ncol_r, &Vp, &taup, &dp, &ep, &ring, &abortp};
+                void* args[] = {&Ac, &n, &ncol_r, &Vp, &taup, &dp, &ep, &ring, &abortp, &kstop, &sub};
                 spin_launch(fn, dim3(wg), dim3(ntr), args, (unsigned)lds, s, num_cu);
             };
             // autotuned workgroup count
@@ -1922,14 +2416,16 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
                     }
                     double best = 1e300;
                     for (int c : cand) {
-                        const double us = time_on_stream(s, 2, [&] { run_reg(c); });
+                        const double us = time_on_stream(s, 2, [&] {
+                            refill();
+                            run_reg(c);
+                        });
                         if (us < best) {
                             best = us;
                             w = c;
                         }
                     }
-                    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, s, ws.bar.get(), 64 + 256);
-                    APW_LAUNCH_CHECK();
+                    refill();
                     tune_store(key, w, 0, best);
                 }
             }
@@ -1939,9 +2435,6 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
             // threads (16 waves x 2 row chunks; 8 waves x 4 chunks measured 1.7x slower)
             const int wmin = (n + 7) / 8, wmax = std::min(num_cu, 256);
             int w = wmax;
-            const size_t nring = (size_t)2 * n * n;
-            ws.ring.reserve(2 * nring);
-            double2* ring = reinterpret_cast<double2*>(ws.ring.get());
             auto run_rows = [&](int wg) {
                 int ncol_r = (n + wg - 1) / wg;
                 constexpr int nw = 16;
@@ -1949,13 +2442,8 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
                                    (size_t)2 * nw * sizeof(double);
                 const void* fn = reinterpret_cast<const void*>(k_tridiag_rows<2, 8, nw>);
                 APW_CHECK(ncol_r <= 8 && n <= 64 * 32, "heevx: row-split form cannot take n=%d on %d workgroups", n, wg);
-                hipLaunchKernelGGL(k_fill_ring, dim3((unsigned)std::min<size_t>(1024, (nring + 255) / 256)), dim3(256),
-                                   0, s, ring, nring);
-                APW_LAUNCH_CHECK();
                 APW_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                const double2* Ac = A;
-                unsigned* abortp = barp + 1;
-                void* args[] = {&Ac, &n, &ncol_r, &Vp, &taup, &dp, &ep, &ring, &abortp};
+                void* args[] = {&Ac, &n, &ncol_r, &Vp, &taup, &dp, &ep, &ring, &abortp, &kstop, &sub};
                 spin_launch(fn, dim3(wg), dim3(64 * nw), args, (unsigned)lds, s, num_cu);
             };
             const int tmode = tune_mode();
@@ -1973,14 +2461,16 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
                     }
                     double best = 1e300;
                     for (int c : cand) {
-                        const double us = time_on_stream(s, 2, [&] { run_rows(c); });
+                        const double us = time_on_stream(s, 2, [&] {
+                            refill();
+                            run_rows(c);
+                        });
                         if (us < best) {
                             best = us;
                             w = c;
                         }
                     }
-                    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, s, ws.bar.get(), 64 + 256);
-                    APW_LAUNCH_CHECK();
+                    refill();
                     tune_store(key, w, 0, best);
                 }
             }
@@ -1988,25 +2478,30 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
         } else {
             // columns in LDS when the share fits, else in A itself (one column per
             // workgroup slot, L2/Infinity-Cache resident); the ring as above
+            int nwg = -1, ncol = 0;
+            for (int w = std::max(1, std::min(n / 8, 16)); w <= std::min(num_cu, 256); ++w) {
+                const int nc = (n + w - 1) / w;
+                if (fixed + (size_t)nc * n * sizeof(double2) <= TRIDIAG_LDS_BYTES) {
+                    nwg = w;
+                    ncol = nc;
+                    break;
+                }
+            }
             const bool gcol = nwg <= 0;
             if (gcol) {
                 nwg = std::min(num_cu, 256);
                 ncol = (n + nwg - 1) / nwg;
             }
             const size_t lds = gcol ? fixed : fixed + (size_t)ncol * n * sizeof(double2);
-            const size_t nring = (size_t)2 * n * (n - 1);
-            ws.ring.reserve(2 * nring);
-            double2* ring = reinterpret_cast<double2*>(ws.ring.get());
-            hipLaunchKernelGGL(k_fill_ring, dim3((unsigned)std::min<size_t>(1024, (nring + 255) / 256)), dim3(256), 0, s,
-                               ring, nring);
-            APW_LAUNCH_CHECK();
             const void* fn = gcol ? reinterpret_cast<const void*>(k_tridiag_fused<true>)
                                   : reinterpret_cast<const void*>(k_tridiag_fused<false>);
             APW_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            unsigned* abortp = barp + 1;
             void* args[] = {&A, &n, &ncol, &Vp, &taup, &dp, &ep, &ring, &abortp};
             spin_launch(fn, dim3(nwg), dim3(NT), args, (unsigned)lds, s, num_cu);
         }
+        if (xcd)
+            tridiag_xcd(s, num_cu, kstop ? sub : Ac, ns, Vp + (size_t)kstop * n + kstop, n, taup + kstop, dp + kstop,
+                        ep + kstop, ring + nring_dev, abortp, joinp);
     } else {
         // n == 1: T = [Re a00]; the real part is the first double of A
         APW_HIP(hipMemcpyAsync(ws.d.get(), A, sizeof(double), hipMemcpyDeviceToDevice, s));
