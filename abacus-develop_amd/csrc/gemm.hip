@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "apw_internal.hpp"
+#include "zgemm_pipe.hpp"
 
 namespace apw {
 namespace {
@@ -405,6 +406,17 @@ void launch(ProfScope& ps, hipStream_t s, int splits, int M, int N, int K, int k
                        reinterpret_cast<c_t*>(C), ldc, ar, ai, br, bi, reinterpret_cast<c_t*>(part));
 }
 
+template <int TA, int TB>
+void launch_pipe(ProfScope& ps, hipStream_t s, int map, int splits, int M, int N, int K, int kchunk, const double* A,
+                 int lda, const double* B, int ldb, double* C, int ldc, double ar, double ai, double br, double bi,
+                 double* part) {
+    const int tm = (M + ZP_BM - 1) / ZP_BM, tn = (N + ZP_BN - 1) / ZP_BN;
+    const dim3 grid = map == 1 ? dim3((unsigned)(((tm + 7) / 8) * 8 * tn), 1, splits) : dim3(tm, tn, splits);
+    APW_PLAUNCH(ps, (zgemm_pipe<TA, TB>), grid, dim3(ZP_NT), 0, s, M, N, K, kchunk, map,
+                reinterpret_cast<const double2*>(A), lda, reinterpret_cast<const double2*>(B), ldb,
+                reinterpret_cast<double2*>(C), ldc, ar, ai, br, bi, reinterpret_cast<double2*>(part));
+}
+
 // R: MFMA type; S: storage type of A, B, C (S = R, or R = float on S = double, see zgemm_kernel)
 template <class R, class S>
 void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, int m, int n, int k,
@@ -433,14 +445,18 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     // 7: 64 x 32, XCD-aware split-K (the tiles of one k split share one XCD's L2); 8: 128 x 64
     // and 9: 128 x 32 with whole m-tiles per XCD and a k step of 16 (half the barriers); 10: 64 x 64
     // with a k step of 16 and 11: the same XCD-aware (split-K candidates: each staged column
-    // of a k-contiguous operand is 256 bytes instead of 128).
+    // of a k-contiguous operand is 256 bytes instead of 128).  FP64 products of 16-byte aligned
+    // operands run the pipelined kernel instead: 12 m-major, 13 with whole m-tiles per XCD (and
+    // 0 when an operand is only 8-byte aligned, which its LDS loads are not written for).
     // occ > 0 splits k so that every workgroup of the launch is resident at once (occ
     // workgroups per CU: floor of the resident slots over the tiles, at least 64 of k per
     // split; a launch with a partial last round of workgroups ran up to 1.5x longer); occ = 0
     // does not split.
-    static const int VBM[12] = {64, 64, 128, 128, 128, 64, 64, 64, 128, 128, 64, 64};
-    static const int VBN[12] = {64, 32, 64, 64, 32, 128, 64, 32, 64, 32, 64, 64};
-    static const int VOCC[12] = {3, 6, 3, 3, 3, 2, 3, 6, 1, 1, 2, 2};   // resident workgroups per CU
+    constexpr bool F64 = std::is_same<R, double>::value;
+    const bool pipe = F64 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0;
+    static const int VBM[14] = {64, 64, 128, 128, 128, 64, 64, 64, 128, 128, 64, 64, ZP_BM, ZP_BM};
+    static const int VBN[14] = {64, 32, 64, 64, 32, 128, 64, 32, 64, 32, 64, 64, ZP_BN, ZP_BN};
+    static const int VOCC[14] = {3, 6, 3, 3, 3, 2, 3, 6, 1, 1, 2, 2, ZP_OCC, ZP_OCC};   // resident workgroups per CU
     const int cus = std::max(num_cu, 64);
     auto tiles_of = [&](int bm, int bn) { return (long)((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
     auto splits_of = [&](int v, int occ) {
@@ -454,14 +470,17 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     };
     const bool tall = m >= 4 * n && m >= 256, wide = n >= 4 * m && n >= 256;
     const bool inner = tiles_of(64, 64) < 2 * cus && k / 64 > 1;
-    // Fixed rule (measured on the Davidson shapes): inner products (k >> m n) split over k
-    // with 64 x 32 tiles when they cover n with fewer columns than 64 x 64 ones (n <= 32,
-    // 65..96), else 64 x 64; tall updates 128 x 32 in the XCD-aware order (with three
-    // accumulator sets the 128 x 64 tile runs one wave per SIMD and lost: 7.1 vs 6.6 ms on
-    // 228487 x 256 x 1024; 64 x 64 made the 216-atom solve 3 % slower); wide 64 x 128; else
-    // 64 x 64.
+    // Fixed rule (measured on the Davidson shapes).  FP64: split over k when the tiles leave
+    // CUs idle; else whole m-tiles per XCD when three or more n-tiles share the rows of A
+    // (228487 x 256 x 1024: 5.33 ms, m-major 5.94), m-major below that, where the narrow last
+    // n-tiles then come last and even out the end (51627 x 97 x 480: 293 us, per XCD 320).
+    // FP32 and x32: inner products (k >> m n) split over k with 64 x 32 tiles when they cover n
+    // with fewer columns than 64 x 64 ones (n <= 32, 65..96), else 64 x 64; tall updates
+    // 128 x 32 in the XCD-aware order; wide 64 x 128; else 64 x 64.
     int variant, occ = 0;
-    if (inner) variant = (n <= 32 || (n > 64 && n <= 96)) ? 1 : 0;
+    if (pipe) variant = !inner && tall && n > 2 * ZP_BN ? 13 : 12;
+    else if (F64) variant = 0;
+    else if (inner) variant = (n <= 32 || (n > 64 && n <= 96)) ? 1 : 0;
     else if (tall) variant = 4;
     else variant = wide ? 5 : 0;
     if (inner) occ = VOCC[variant];
@@ -498,39 +517,41 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
             ProfScope ps(pf, s, pname,
                          esz * ((double)m * k + (double)k * n + (double)m * n * (splits > 1 ? splits : (beta_nz ? 2 : 1))),
                          8.0 * m * n * (double)k, true);
+#define APW_GEMM_TILE(V, X, Y, TM, TN, BK, MAP)                                                                      \
+    case V: launch<R, S, X, Y, TM, TN, BK, MAP>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re,   \
+                                                alpha_im, b_re, b_im, part); break;
 #define APW_GEMM_CASE(X, Y)                                                                                          \
-    if (oa == X && ob == Y) {                                                                                       \
-        switch (v) {                                                                                                \
-            case 1: launch<R, S, X, Y, 2, 1, 8, 0>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                               alpha_im, b_re, b_im, part); break;                                  \
-            case 2: launch<R, S, X, Y, 4, 2, 8, 1>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                               alpha_im, b_re, b_im, part); break;                                  \
-            case 3: launch<R, S, X, Y, 4, 2, 8, 2>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                               alpha_im, b_re, b_im, part); break;                                  \
-            case 4: launch<R, S, X, Y, 4, 1, 8, 2>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                               alpha_im, b_re, b_im, part); break;                                  \
-            case 5: launch<R, S, X, Y, 2, 4, 16, 0>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                                alpha_im, b_re, b_im, part); break;                                 \
-            case 6: launch<R, S, X, Y, 2, 2, 8, 3>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                               alpha_im, b_re, b_im, part); break;                                  \
-            case 7: launch<R, S, X, Y, 2, 1, 8, 3>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                               alpha_im, b_re, b_im, part); break;                                  \
-            case 8: launch<R, S, X, Y, 4, 2, 16, 2>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                                alpha_im, b_re, b_im, part); break;                                 \
-            case 9: launch<R, S, X, Y, 4, 1, 16, 2>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                                alpha_im, b_re, b_im, part); break;                                 \
-            case 10: launch<R, S, X, Y, 2, 2, 16, 0>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                                 alpha_im, b_re, b_im, part); break;                                \
-            case 11: launch<R, S, X, Y, 2, 2, 16, 3>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                                 alpha_im, b_re, b_im, part); break;                                \
-            default: launch<R, S, X, Y, 2, 2, 8, 0>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re, \
-                                                alpha_im, b_re, b_im, part); break;                                 \
-        }                                                                                                           \
+    if (oa == X && ob == Y) {                                                                                        \
+        if constexpr (F64) {                                                                                         \
+            if (v >= 12)                                                                                             \
+                launch_pipe<X, Y>(ps, s, v - 12, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re,        \
+                                  alpha_im, b_re, b_im, part);                                                       \
+            else                                                                                                     \
+                launch<R, S, X, Y, 2, 2, 8, 0>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re,   \
+                                               alpha_im, b_re, b_im, part);                                          \
+        } else {                                                                                                     \
+            switch (v) {                                                                                             \
+                APW_GEMM_TILE(1, X, Y, 2, 1, 8, 0)                                                                   \
+                APW_GEMM_TILE(2, X, Y, 4, 2, 8, 1)                                                                   \
+                APW_GEMM_TILE(3, X, Y, 4, 2, 8, 2)                                                                   \
+                APW_GEMM_TILE(4, X, Y, 4, 1, 8, 2)                                                                   \
+                APW_GEMM_TILE(5, X, Y, 2, 4, 16, 0)                                                                  \
+                APW_GEMM_TILE(6, X, Y, 2, 2, 8, 3)                                                                   \
+                APW_GEMM_TILE(7, X, Y, 2, 1, 8, 3)                                                                   \
+                APW_GEMM_TILE(8, X, Y, 4, 2, 16, 2)                                                                  \
+                APW_GEMM_TILE(9, X, Y, 4, 1, 16, 2)                                                                  \
+                APW_GEMM_TILE(10, X, Y, 2, 2, 16, 0)                                                                 \
+                APW_GEMM_TILE(11, X, Y, 2, 2, 16, 3)                                                                 \
+                default: launch<R, S, X, Y, 2, 2, 8, 0>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp,    \
+                                                        alpha_re, alpha_im, b_re, b_im, part); break;                \
+            }                                                                                                        \
+        }                                                                                                            \
     }
             APW_GEMM_CASE(0, 0) APW_GEMM_CASE(0, 1) APW_GEMM_CASE(0, 2)
             APW_GEMM_CASE(1, 0) APW_GEMM_CASE(1, 1) APW_GEMM_CASE(1, 2)
             APW_GEMM_CASE(2, 0) APW_GEMM_CASE(2, 1) APW_GEMM_CASE(2, 2)
 #undef APW_GEMM_CASE
+#undef APW_GEMM_TILE
             APW_LAUNCH_CHECK();
         }
         if (splits > 1) {
@@ -546,21 +567,26 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     };
     // autotuned plan (the fixed-workspace entry point keeps the fixed rule, whose partials
     // it is sized for)
-    const int tmode = ws.ext ? 0 : tune_mode();
+    const int tmode = ws.ext || (F64 && !pipe) ? 0 : tune_mode();
     if (tmode > 0) {
         auto bucket = [](int x) { return x <= 2048 ? (x + 31) / 32 * 32 : (x + 1023) / 1024 * 1024; };
         char key[160];
         std::snprintf(key, sizeof(key), "gemm %s %c%c m=%d n=%d k=%d cu=%d", prec_tag, "NTC"[oa], "NTC"[ob],
                       bucket(m), bucket(n), bucket(k), cus);
         int a = 0, b = 0;
-        if (tune_find(key, a, b) && a >= 0 && a < 12 && b >= 0 && b <= 6 && !(X32 && (a == 2 || a == 3 || a == 8))) {
+        const int lo = F64 ? 12 : 0, hi = F64 ? 14 : 12;   // variants this precision has
+        if (tune_find(key, a, b) && a >= lo && a < hi && b >= 0 && b <= 6 && !(X32 && (a == 2 || a == 3 || a == 8))) {
             variant = a;
             occ = b;
         } else if (tmode == 2) {
             // candidates: every tile/map of the shape's kind, and for inner products every
             // split rule; timed into a scratch C (beta 0) so the caller's C is untouched
             std::vector<std::pair<int, int>> cand;
-            if (inner) {
+            if (F64) {
+                for (int oc : {1, 2, 3})
+                    if (inner) cand.emplace_back(12, oc);
+                if (!inner) cand = {{12, 0}, {13, 0}};
+            } else if (inner) {
                 for (int v : {0, 1, 6, 7, 10, 11})
                     for (int oc : {1, 2, 3, 4, 6}) cand.emplace_back(v, oc);
             } else if (tall) {
