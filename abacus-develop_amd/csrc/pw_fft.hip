@@ -703,12 +703,19 @@ __global__ __launch_bounds__(xreg_threads(N)) void k_xreg(cplx<R>* __restrict__ 
 }
 
 // ---- density pass, register form: rho (+)= sum_b w_b |x-backward(psi_b)|^2 ------------
-// grid (ny, ceil(nz / XL)); bands in order inside the workgroup, sums in registers.
+// grid (ny, ceil(nz / XL)); bands in order inside the workgroup, sums in registers.  Bound by
+// the reads of X, once enough waves are resident to cover a band's chain of load, transform,
+// exchange and transform: the sums and step B leave 168 registers for three waves a SIMD only
+// when the twiddles are read again for each band (a 256-byte table in the vector cache) and no
+// loads are kept for the next band, which the other waves' work hides better (four bands of
+// 160^3, 75 slots: 56.9 -> 44.1 us, 4.3 TB/s, what a large copy reaches; both kept: two waves
+// a SIMD; prefetch and twiddles in LDS 49.1; four waves a SIMD spill: 70.1).
 template <int N>
-__global__ __launch_bounds__(xreg_threads(N)) void k_xrho_reg(const cplx<double>* __restrict__ X, int nxr, int ny,
-                                                             int nz, int nb, int4 xrun, const double* __restrict__ w,
-                                                             double* __restrict__ rho, int add,
-                                                             const cplx<double>* __restrict__ tw) {
+__global__ __launch_bounds__(xreg_threads(N), 3) void k_xrho_reg(const cplx<double>* __restrict__ X, int nxr, int ny,
+                                                                int nz, int nb, int4 xrun,
+                                                                const double* __restrict__ w,
+                                                                double* __restrict__ rho, int add,
+                                                                const cplx<double>* __restrict__ tw) {
     using C = cplx<double>;
     constexpr int NA = ct_split_a(N), NB = N / NA;
     __shared__ C buf[N * XL];
@@ -718,31 +725,23 @@ __global__ __launch_bounds__(xreg_threads(N)) void k_xrho_reg(const cplx<double>
     const size_t plane = (size_t)ny * nz, off = (size_t)iy * nz + (zin ? iz : 0);
     const bool mid = g < NA;
     unsigned qo[NA];
-    C twa[NA];
     static_for<0, NA>([&](auto n1) {
         const int q = xrun_slot(xrun, NB * APW_CI(n1) + g);
         qo[APW_CI(n1)] = (zin && q >= 0) ? (unsigned)(((size_t)q * plane + off) * sizeof(C)) : BUF_OOB;
     });
-    static_for<0, NA>([&](auto k1) {
-        C t = tw[g * APW_CI(k1)];
-        t.y = -t.y;
-        twa[APW_CI(k1)] = t;
-    });
     double acc[NB];
     static_for<0, NB>([&](auto k2) { acc[APW_CI(k2)] = 0.0; });
-    C v[NA], vn[NA], u[NB];
     const unsigned band_bytes = (unsigned)(nxr * plane * sizeof(C));
-    if (nb > 0) {
-        const __amdgpu_buffer_rsrc_t xr = make_rsrc(X, band_bytes);
-        static_for<0, NA>([&](auto n1) { v[APW_CI(n1)] = buf_load(xr, qo[APW_CI(n1)], (C*)nullptr); });
-    }
     for (int b = 0; b < nb; ++b) {
-        if (b + 1 < nb) {   // the next band's loads fly while this band is transformed
-            const __amdgpu_buffer_rsrc_t xr = make_rsrc(X + (size_t)(b + 1) * nxr * plane, band_bytes);
-            static_for<0, NA>([&](auto n1) { vn[APW_CI(n1)] = buf_load(xr, qo[APW_CI(n1)], (C*)nullptr); });
-        }
+        C v[NA], u[NB];
+        const __amdgpu_buffer_rsrc_t xr = make_rsrc(X + (size_t)b * nxr * plane, band_bytes);
+        static_for<0, NA>([&](auto n1) { v[APW_CI(n1)] = buf_load(xr, qo[APW_CI(n1)], (C*)nullptr); });
         rdft<C, double, NA, +1>(v);
-        static_for<1, NA>([&](auto k1) { v[APW_CI(k1)] = cmul(v[APW_CI(k1)], twa[APW_CI(k1)]); });
+        static_for<1, NA>([&](auto k1) {
+            C t = tw[g * APW_CI(k1)];   // g k1 < N
+            t.y = -t.y;
+            v[APW_CI(k1)] = cmul(v[APW_CI(k1)], t);
+        });
         __syncthreads();   // the previous band's reads of buf are done
         static_for<0, NA>([&](auto k1) { buf[(APW_CI(k1) * NB + g) * XL + l] = v[APW_CI(k1)]; });
         __syncthreads();
@@ -755,7 +754,6 @@ __global__ __launch_bounds__(xreg_threads(N)) void k_xrho_reg(const cplx<double>
                 acc[APW_CI(k2)] += wb * (r.x * r.x + r.y * r.y);
             });
         }
-        static_for<0, NA>([&](auto n1) { v[APW_CI(n1)] = vn[APW_CI(n1)]; });
     }
     if (mid && zin) {
         static_for<0, NB>([&](auto k2) {
