@@ -7,9 +7,12 @@
 //   * update shapes         C(npw x n) += A(npw x k) B(k x n) with k <= ~2e3
 //     (back-projection, cal_grad, refresh, final psi) -> plain 2D tiling.
 //
-// Tile: 64 x 64, 128 x 64 or 64 x 128 (m x n) per workgroup, k step 8 (16 for the wide
-// tile) through two LDS stages, 4 waves in a 2 x 2 arrangement, each wave owning TM x TN MFMA 16x16 sub-tiles
-// with separate accumulators (a complex product = 3 real MFMAs; 4 in the x32 form).  Operand roles are swapped
+// The FP64 and FP32 products run the pipelined tile of zgemm_pipe.hpp (a complex product = 3
+// real MFMAs); this file holds the x32 form (c128 operands rounded to FP32 on their way to LDS,
+// which a direct fill cannot do; 4 real MFMAs), the split-K reduction and the choice of plan.
+// x32 tile: 64 x 32 to 128 x 32 or 64 x 128 (m x n) per workgroup, k step 8 or 16 through two LDS
+// stages, 4 waves in a 2 x 2 arrangement, each wave owning TM x TN MFMA 16x16 sub-tiles
+// with separate accumulators.  Operand roles are swapped
 // (MFMA "A" <- op(B) indexed by n, MFMA "B" <- op(A) indexed by m) so that the 16 lanes of
 // a group hold 16 consecutive rows m of one column n: the column-major stores of C are then
 // 256-byte coalesced runs.  Accumulator register r of lane l holds D row drow(l, r) and
@@ -61,27 +64,20 @@ constexpr int BKMAX = 16, NT = 256;
 // after the next is loaded into registers and the next one is written to stage s^1, so a
 // k step costs one workgroup barrier.  LDS rows are padded (16 / BK elements) so that the
 // k-fastest operand stores fall in distinct banks.
-// S: element type of A, B, C and the split-K partials.  S = R is the plain form.  R = float
-// with S = double is the FP32-MFMA form of an FP64 product: operands rounded to FP32 as
-// they are staged in LDS, FP32 accumulators folded into FP64 ones every XFOLD k steps
-// (32 or 64 k values), so the rounding is that of the FP32 operands, not of a long FP32
-// sum; C and the partials stay FP64.
+// FP32-MFMA form of an FP64 product: operands rounded to FP32 as they are staged in LDS, FP32
+// accumulators folded into FP64 ones every XFOLD k steps (32 or 64 k values), so the rounding
+// is that of the FP32 operands, not of a long FP32 sum; A, B, C and the split-K partials are FP64.
 constexpr int XFOLD = 4;
-template <class R, class S, int TA, int TB, int TM, int TN, int BK, int MAP>
+template <int TA, int TB, int TM, int TN, int BK, int MAP>
 __global__ __launch_bounds__(NT) void zgemm_kernel(int M, int N, int K, int kchunk,
-                                                   const typename Mfma<S>::c_t* __restrict__ A, int lda,
-                                                   const typename Mfma<S>::c_t* __restrict__ B, int ldb,
-                                                   typename Mfma<S>::c_t* __restrict__ C, int ldc,
+                                                   const double2* __restrict__ A, int lda,
+                                                   const double2* __restrict__ B, int ldb,
+                                                   double2* __restrict__ C, int ldc,
                                                    double ar, double ai, double br, double bi,
-                                                   typename Mfma<S>::c_t* __restrict__ part) {
-    using c_t = typename Mfma<S>::c_t;
-    using acc_t = typename Mfma<R>::acc_t;
-    constexpr bool X32 = !std::is_same<R, S>::value;
-    static_assert(!X32 || (std::is_same<R, float>::value && std::is_same<S, double>::value), "x32: f32 on f64");
-    // three real products per complex one (P1 = re re, P2 = im im, P3 = (re + im)(re + im);
-    // re = P1 - P2, im = P3 - P1 - P2), 3 MFMAs instead of 4; the error stays normwise, a few
-    // ulps of |a||b| per term.  The x32 form keeps four (its FP32 sums are folded into FP64)
-    constexpr bool M3 = !X32;
+                                                   double2* __restrict__ part) {
+    using R = float;
+    using c_t = double2;
+    using acc_t = Mfma<R>::acc_t;
     constexpr int BM = 32 * TM, BN = 32 * TN;
     constexpr int NA = BM * BK / NT, NB = BN * BK / NT;
     // row padding 16 / BK elements: a k-fastest staging store puts 16 lanes on BK consecutive
@@ -96,7 +92,7 @@ __global__ __launch_bounds__(NT) void zgemm_kernel(int M, int N, int K, int kchu
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int wm = wave & 1, wn = wave >> 1;
-    // tile of this workgroup.  MAP 0: blockIdx.x walks m; MAP 1: it walks n.  MAP 2 (XCD-aware,
+    // tile of this workgroup.  MAP 0: blockIdx.x walks m.  MAP 2 (XCD-aware,
     // 1-D grid in x; measured slower for split-K, used for the tall updates only):
     // workgroup L runs on XCD L % 8, so each XCD takes whole m-tiles and walks their n-tiles
     // back to back; the A tile they share stays in that XCD's L2.  The grid is padded to a
@@ -106,10 +102,7 @@ __global__ __launch_bounds__(NT) void zgemm_kernel(int M, int N, int K, int kchu
     // at the same k come from that XCD's L2 instead of once per tile from HBM.  XCD x takes
     // the x-th eighth of the (split, tile) sequence, tiles of a split consecutive.
     int bm = blockIdx.x, bn = blockIdx.y, sp = blockIdx.z;
-    if (MAP == 1) {   // blockIdx.x walks n
-        bm = blockIdx.y;
-        bn = blockIdx.x;
-    } else if (MAP == 2) {
+    if (MAP == 2) {
         const int L = blockIdx.x;
         const int ntn = (N + BN - 1) / BN, tmt = (M + BM - 1) / BM;
         bm = (L % 8) + 8 * (L / (8 * ntn));
@@ -129,36 +122,30 @@ __global__ __launch_bounds__(NT) void zgemm_kernel(int M, int N, int K, int kchu
     const int kbeg = sp * kchunk;
     const int kend = min(K, kbeg + kchunk);
 
-    acc_t acc_re[TN][TM], acc_im[TN][TM];   // 4M: re, im; 3M: P1, P3
-    acc_t acc_p2[M3 ? TN : 1][M3 ? TM : 1];   // 3M: P2
-    d4_t wide_re[X32 ? TN : 1][X32 ? TM : 1], wide_im[X32 ? TN : 1][X32 ? TM : 1];   // X32: FP64 sums
+    acc_t acc_re[TN][TM], acc_im[TN][TM];
+    d4_t wide_re[TN][TM], wide_im[TN][TM];   // FP64 sums
 #pragma unroll
     for (int a = 0; a < TN; ++a)
 #pragma unroll
         for (int b = 0; b < TM; ++b) {
             acc_re[a][b] = acc_t{0, 0, 0, 0};
             acc_im[a][b] = acc_t{0, 0, 0, 0};
-            if constexpr (M3) acc_p2[a][b] = acc_t{0, 0, 0, 0};
-            if constexpr (X32) {
-                wide_re[a][b] = d4_t{0, 0, 0, 0};
-                wide_im[a][b] = d4_t{0, 0, 0, 0};
-            }
+            wide_re[a][b] = d4_t{0, 0, 0, 0};
+            wide_im[a][b] = d4_t{0, 0, 0, 0};
         }
     auto fold = [&]() {
-        if constexpr (X32) {
 #pragma unroll
-            for (int a = 0; a < TN; ++a)
+        for (int a = 0; a < TN; ++a)
 #pragma unroll
-                for (int b = 0; b < TM; ++b) {
+            for (int b = 0; b < TM; ++b) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        wide_re[a][b][r] += (double)acc_re[a][b][r];
-                        wide_im[a][b][r] += (double)acc_im[a][b][r];
-                    }
-                    acc_re[a][b] = acc_t{0, 0, 0, 0};
-                    acc_im[a][b] = acc_t{0, 0, 0, 0};
+                for (int r = 0; r < 4; ++r) {
+                    wide_re[a][b][r] += (double)acc_re[a][b][r];
+                    wide_im[a][b][r] += (double)acc_im[a][b][r];
                 }
-        }
+                acc_re[a][b] = acc_t{0, 0, 0, 0};
+                acc_im[a][b] = acc_t{0, 0, 0, 0};
+            }
     };
 
     // Prefetch registers.  The loads are unconditional (an out-of-range element reads
@@ -246,41 +233,23 @@ __global__ __launch_bounds__(NT) void zgemm_kernel(int M, int N, int K, int kchu
                 yr[t] = As[st][0][kk][mm];
                 yi[t] = As[st][1][kk][mm];
             }
-            if constexpr (M3) {
-                R xs[TN], ys[TM];
 #pragma unroll
-                for (int t = 0; t < TN; ++t) xs[t] = xr[t] + xi[t];
+            for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-                for (int t = 0; t < TM; ++t) ys[t] = yr[t] + yi[t];
-#pragma unroll
-                for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-                    for (int tm = 0; tm < TM; ++tm) {
-                        acc_re[tn][tm] = Mfma<R>::mma(xr[tn], yr[tm], acc_re[tn][tm]);
-                        acc_p2[tn][tm] = Mfma<R>::mma(xi[tn], yi[tm], acc_p2[tn][tm]);
-                        acc_im[tn][tm] = Mfma<R>::mma(xs[tn], ys[tm], acc_im[tn][tm]);
-                    }
-            } else {
-#pragma unroll
-                for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-                    for (int tm = 0; tm < TM; ++tm) {
-                        acc_re[tn][tm] = Mfma<R>::mma(xr[tn], yr[tm], acc_re[tn][tm]);
-                        acc_re[tn][tm] = Mfma<R>::mma(-xi[tn], yi[tm], acc_re[tn][tm]);
-                        acc_im[tn][tm] = Mfma<R>::mma(xr[tn], yi[tm], acc_im[tn][tm]);
-                        acc_im[tn][tm] = Mfma<R>::mma(xi[tn], yr[tm], acc_im[tn][tm]);
-                    }
-            }
+                for (int tm = 0; tm < TM; ++tm) {
+                    acc_re[tn][tm] = Mfma<R>::mma(xr[tn], yr[tm], acc_re[tn][tm]);
+                    acc_re[tn][tm] = Mfma<R>::mma(-xi[tn], yi[tm], acc_re[tn][tm]);
+                    acc_im[tn][tm] = Mfma<R>::mma(xr[tn], yi[tm], acc_im[tn][tm]);
+                    acc_im[tn][tm] = Mfma<R>::mma(xi[tn], yr[tm], acc_im[tn][tm]);
+                }
         }
         // unconditional (one basic block with the MFMAs): past the end the masks are zero and
         // the loads read element 0
         stage(st ^ 1);
         fetch(k0 + 2 * BK);
-        if constexpr (X32) {
-            if (++nfold == XFOLD) {
-                fold();
-                nfold = 0;
-            }
+        if (++nfold == XFOLD) {
+            fold();
+            nfold = 0;
         }
         __syncthreads();
         st ^= 1;
@@ -297,22 +266,11 @@ __global__ __launch_bounds__(NT) void zgemm_kernel(int M, int N, int K, int kchu
                 const int gm = m0 + wm * 16 * TM + tm * 16 + (lane & 15);
                 const int gn = n0 + wn * 16 * TN + tn * 16 + Mfma<R>::drow(lane, r);
                 if (gm >= M || gn >= N) continue;
-                double xr, xi;
-                if constexpr (X32) {
-                    xr = wide_re[tn][tm][r];
-                    xi = wide_im[tn][tm][r];
-                } else if constexpr (M3) {
-                    const double p1 = acc_re[tn][tm][r], p2 = acc_p2[tn][tm][r];
-                    xr = p1 - p2;
-                    xi = (double)acc_im[tn][tm][r] - (p1 + p2);
-                } else {
-                    xr = (double)acc_re[tn][tm][r];
-                    xi = (double)acc_im[tn][tm][r];
-                }
+                const double xr = wide_re[tn][tm][r], xi = wide_im[tn][tm][r];
                 if (part) {
                     c_t v;
-                    v.x = (S)xr;
-                    v.y = (S)xi;
+                    v.x = xr;
+                    v.y = xi;
                     part[(size_t)sp * M * N + gm + (size_t)gn * M] = v;
                 } else {
                     double cr = ar * xr - ai * xi;
@@ -320,12 +278,12 @@ __global__ __launch_bounds__(NT) void zgemm_kernel(int M, int N, int K, int kchu
                     c_t* cp = C + gm + (size_t)gn * ldc;
                     if (br != 0.0 || bi != 0.0) {
                         const c_t c = *cp;
-                        cr += br * (double)c.x - bi * (double)c.y;
-                        ci += br * (double)c.y + bi * (double)c.x;
+                        cr += br * c.x - bi * c.y;
+                        ci += br * c.y + bi * c.x;
                     }
                     c_t v;
-                    v.x = (S)cr;
-                    v.y = (S)ci;
+                    v.x = cr;
+                    v.y = ci;
                     *cp = v;
                 }
             }
@@ -419,31 +377,31 @@ int opcode(char t) {
     }
 }
 
-template <class R, class S, int TA, int TB, int TM, int TN, int BK, int MAP>
-void launch(ProfScope& ps, hipStream_t s, int splits, int M, int N, int K, int kchunk, const S* A, int lda,
-            const S* B, int ldb, S* C, int ldc, double ar, double ai, double br, double bi, S* part) {
-    using c_t = typename Mfma<S>::c_t;
+template <int TA, int TB, int TM, int TN, int BK, int MAP>
+void launch_x32(ProfScope& ps, hipStream_t s, int splits, int M, int N, int K, int kchunk, const double* A, int lda,
+                const double* B, int ldb, double* C, int ldc, double ar, double ai, double br, double bi,
+                double* part) {
     const int tm = (M + 32 * TM - 1) / (32 * TM), tn = (N + 32 * TN - 1) / (32 * TN);
     const dim3 grid = MAP == 3   ? dim3((unsigned)((tm * tn * splits + 7) / 8 * 8), 1, 1)
                       : MAP == 2 ? dim3((unsigned)(((tm + 7) / 8) * 8 * tn), 1, splits)
-                                 : (MAP == 1 ? dim3(tn, tm, splits) : dim3(tm, tn, splits));
-    APW_PLAUNCH(ps, (zgemm_kernel<R, S, TA, TB, TM, TN, BK, MAP>), grid, dim3(NT), 0, s, M, N, K, kchunk,
-                       reinterpret_cast<const c_t*>(A), lda, reinterpret_cast<const c_t*>(B), ldb,
-                       reinterpret_cast<c_t*>(C), ldc, ar, ai, br, bi, reinterpret_cast<c_t*>(part));
-}
-
-template <int TA, int TB>
-void launch_pipe(ProfScope& ps, hipStream_t s, int map, int splits, int M, int N, int K, int kchunk, const double* A,
-                 int lda, const double* B, int ldb, double* C, int ldc, double ar, double ai, double br, double bi,
-                 double* part) {
-    const int tm = (M + ZP_BM - 1) / ZP_BM, tn = (N + ZP_BN - 1) / ZP_BN;
-    const dim3 grid = map == 1 ? dim3((unsigned)(((tm + 7) / 8) * 8 * tn), 1, splits) : dim3(tm, tn, splits);
-    APW_PLAUNCH(ps, (zgemm_pipe<TA, TB>), grid, dim3(ZP_NT), 0, s, M, N, K, kchunk, map,
+                                 : dim3(tm, tn, splits);
+    APW_PLAUNCH(ps, (zgemm_kernel<TA, TB, TM, TN, BK, MAP>), grid, dim3(NT), 0, s, M, N, K, kchunk,
                 reinterpret_cast<const double2*>(A), lda, reinterpret_cast<const double2*>(B), ldb,
                 reinterpret_cast<double2*>(C), ldc, ar, ai, br, bi, reinterpret_cast<double2*>(part));
 }
 
-// R: MFMA type; S: storage type of A, B, C (S = R, or R = float on S = double, see zgemm_kernel)
+template <class R, int TA, int TB>
+void launch_pipe(ProfScope& ps, hipStream_t s, int map, int splits, int M, int N, int K, int kchunk, const R* A,
+                 int lda, const R* B, int ldb, R* C, int ldc, double ar, double ai, double br, double bi, R* part) {
+    using c_t = typename ZpType<R>::c_t;
+    const int tm = (M + ZP_BM - 1) / ZP_BM, tn = (N + ZP_BN - 1) / ZP_BN;
+    const dim3 grid = map == 1 ? dim3((unsigned)(((tm + 7) / 8) * 8 * tn), 1, splits) : dim3(tm, tn, splits);
+    APW_PLAUNCH(ps, (zgemm_pipe<R, TA, TB>), grid, dim3(ZP_NT), 0, s, M, N, K, kchunk, map,
+                reinterpret_cast<const c_t*>(A), lda, reinterpret_cast<const c_t*>(B), ldb,
+                reinterpret_cast<c_t*>(C), ldc, ar, ai, br, bi, reinterpret_cast<c_t*>(part));
+}
+
+// R: MFMA type; S: storage type of A, B, C (S = R, or R = float on S = double: the x32 form)
 template <class R, class S>
 void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, int m, int n, int k,
                double alpha_re, double alpha_im, const S* A, int lda, const S* B, int ldb,
@@ -465,24 +423,21 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
         APW_LAUNCH_CHECK();
         return;
     }
-    // Plans: a tile variant and a split rule.  Variants (TM x TN MFMA sub-tiles per wave, map):
-    // 0: 64 x 64, m-major; 1: 64 x 32, m-major; 2: 128 x 64, n-major; 3: 128 x 64 and 4: 128 x 32,
-    // XCD-aware (each XCD takes whole m-tiles); 5: 64 x 128 with k step 16; 6: 64 x 64 and
-    // 7: 64 x 32, XCD-aware split-K (the tiles of one k split share one XCD's L2); 8: 128 x 64
-    // and 9: 128 x 32 with whole m-tiles per XCD and a k step of 16 (half the barriers); 10: 64 x 64
-    // with a k step of 16 and 11: the same XCD-aware (split-K candidates: each staged column
-    // of a k-contiguous operand is 256 bytes instead of 128).  FP64 products of 16-byte aligned
-    // operands run the pipelined kernel instead: 12 m-major, 13 with whole m-tiles per XCD (and
-    // 0 when an operand is only 8-byte aligned, which its LDS loads are not written for).
+    // Plans: a tile variant and a split rule.  FP64 and FP32 (64 x 64 tiles of zgemm_pipe.hpp):
+    // 12 m-major, 13 with whole m-tiles per XCD.  x32 variants (TM x TN MFMA sub-tiles per
+    // wave, map): 0: 64 x 64, m-major; 1: 64 x 32, m-major; 4: 128 x 32, XCD-aware (each XCD takes
+    // whole m-tiles); 5: 64 x 128 with k step 16; 6: 64 x 64 and 7: 64 x 32, XCD-aware split-K (the
+    // tiles of one k split share one XCD's L2); 9: 128 x 32 with whole m-tiles per XCD and a k step
+    // of 16 (half the barriers); 10: 64 x 64 with a k step of 16 and 11: the same XCD-aware
+    // (split-K candidates: each staged column of a k-contiguous operand is 256 bytes, not 128).
     // occ > 0 splits k so that every workgroup of the launch is resident at once (occ
     // workgroups per CU: floor of the resident slots over the tiles, at least 64 of k per
     // split; a launch with a partial last round of workgroups ran up to 1.5x longer); occ = 0
     // does not split.
-    constexpr bool F64 = std::is_same<R, double>::value;
-    const bool pipe = F64 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0;
-    static const int VBM[14] = {64, 64, 128, 128, 128, 64, 64, 64, 128, 128, 64, 64, ZP_BM, ZP_BM};
-    static const int VBN[14] = {64, 32, 64, 64, 32, 128, 64, 32, 64, 32, 64, 64, ZP_BN, ZP_BN};
-    static const int VOCC[14] = {3, 6, 3, 3, 3, 2, 3, 6, 1, 1, 2, 2, ZP_OCC, ZP_OCC};   // resident workgroups per CU
+    static const int VBM[14] = {64, 64, 0, 0, 128, 64, 64, 64, 0, 128, 64, 64, ZP_BM, ZP_BM};
+    static const int VBN[14] = {64, 32, 0, 0, 32, 128, 64, 32, 0, 32, 64, 64, ZP_BN, ZP_BN};
+    static const int VOCC[14] = {3, 6, 0, 0, 3, 2, 3, 6, 0, 1, 2, 2, ZP_OCC, ZP_OCC};   // resident workgroups per CU
+    auto has = [&](int v) { return X32 ? v >= 0 && v < 12 && VBM[v] > 0 : v == 12 || v == 13; };
     const int cus = std::max(num_cu, 64);
     auto tiles_of = [&](int bm, int bn) { return (long)((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
     auto splits_of = [&](int v, int occ) {
@@ -496,20 +451,22 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     };
     const bool tall = m >= 4 * n && m >= 256, wide = n >= 4 * m && n >= 256;
     const bool inner = tiles_of(64, 64) < 2 * cus && k / 64 > 1;
-    // Fixed rule (measured on the Davidson shapes).  FP64: split over k when the tiles leave
-    // CUs idle; else whole m-tiles per XCD when three or more n-tiles share the rows of A
-    // (228487 x 256 x 1024: 5.33 ms, m-major 5.94), m-major below that, where the narrow last
-    // n-tiles then come last and even out the end (51627 x 97 x 480: 293 us, per XCD 320).
-    // FP32 and x32: inner products (k >> m n) split over k with 64 x 32 tiles when they cover n
-    // with fewer columns than 64 x 64 ones (n <= 32, 65..96), else 64 x 64; tall updates
-    // 128 x 32 in the XCD-aware order; wide 64 x 128; else 64 x 64.
+    // Fixed rule (measured on the Davidson shapes): split over k when the tiles leave CUs idle;
+    // else whole m-tiles per XCD where enough n-tiles share the rows of A (c128 three, c64
+    // four: 228487 x 256 x 1024 5.33 ms, m-major 5.94; c64 2.80 and 3.18), m-major below that,
+    // where the narrow last n-tiles then come last and even out the end (51627 x 97 x 480: 293 us,
+    // per XCD 320; c64 51627 x 160 x 512: 219 and 237).  c64 products of few columns are
+    // split twice as often: the sums of a split are FP32.
+    // x32: inner products with 64 x 32 tiles when they cover n with fewer columns than 64 x 64
+    // ones (n <= 32, 65..96), else 64 x 64; tall updates 128 x 32 in the XCD-aware order; wide
+    // 64 x 128; else 64 x 64.
+    const bool few = n <= 32 || (n > 64 && n <= 96);
     int variant, occ = 0;
-    if (pipe) variant = !inner && tall && n > 2 * ZP_BN ? 13 : 12;
-    else if (F64) variant = 0;
-    else if (inner) variant = (n <= 32 || (n > 64 && n <= 96)) ? 1 : 0;
+    if (!X32) variant = !inner && tall && n > (sizeof(S) == 8 ? 2 : 3) * ZP_BN ? 13 : 12;
+    else if (inner) variant = few ? 1 : 0;
     else if (tall) variant = 4;
     else variant = wide ? 5 : 0;
-    if (inner) occ = VOCC[variant];
+    if (inner) occ = (!X32 && sizeof(S) == 4 && few ? 2 : 1) * VOCC[variant];
     const char* prec_tag = X32 ? "x32" : (std::is_same<R, double>::value ? "f64" : "f32");
     auto need_of = [&](int v, int oc) {
         const int sp = splits_of(v, oc);
@@ -544,32 +501,24 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
                          esz * ((double)m * k + (double)k * n + (double)m * n * (splits > 1 ? splits : (beta_nz ? 2 : 1))),
                          8.0 * m * n * (double)k, true);
 #define APW_GEMM_TILE(V, X, Y, TM, TN, BK, MAP)                                                                      \
-    case V: launch<R, S, X, Y, TM, TN, BK, MAP>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re,   \
-                                                alpha_im, b_re, b_im, part); break;
+    case V: launch_x32<X, Y, TM, TN, BK, MAP>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re,     \
+                                              alpha_im, b_re, b_im, part); break;
 #define APW_GEMM_CASE(X, Y)                                                                                          \
     if (oa == X && ob == Y) {                                                                                        \
-        if constexpr (F64) {                                                                                         \
-            if (v >= 12)                                                                                             \
-                launch_pipe<X, Y>(ps, s, v - 12, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re,        \
-                                  alpha_im, b_re, b_im, part);                                                       \
-            else                                                                                                     \
-                launch<R, S, X, Y, 2, 2, 8, 0>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re,   \
-                                               alpha_im, b_re, b_im, part);                                          \
+        if constexpr (!X32) {                                                                                        \
+            launch_pipe<R, X, Y>(ps, s, v - 12, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp, alpha_re,         \
+                                 alpha_im, b_re, b_im, part);                                                        \
         } else {                                                                                                     \
             switch (v) {                                                                                             \
+                APW_GEMM_TILE(0, X, Y, 2, 2, 8, 0)                                                                   \
                 APW_GEMM_TILE(1, X, Y, 2, 1, 8, 0)                                                                   \
-                APW_GEMM_TILE(2, X, Y, 4, 2, 8, 1)                                                                   \
-                APW_GEMM_TILE(3, X, Y, 4, 2, 8, 2)                                                                   \
                 APW_GEMM_TILE(4, X, Y, 4, 1, 8, 2)                                                                   \
                 APW_GEMM_TILE(5, X, Y, 2, 4, 16, 0)                                                                  \
                 APW_GEMM_TILE(6, X, Y, 2, 2, 8, 3)                                                                   \
                 APW_GEMM_TILE(7, X, Y, 2, 1, 8, 3)                                                                   \
-                APW_GEMM_TILE(8, X, Y, 4, 2, 16, 2)                                                                  \
                 APW_GEMM_TILE(9, X, Y, 4, 1, 16, 2)                                                                  \
                 APW_GEMM_TILE(10, X, Y, 2, 2, 16, 0)                                                                 \
                 APW_GEMM_TILE(11, X, Y, 2, 2, 16, 3)                                                                 \
-                default: launch<R, S, X, Y, 2, 2, 8, 0>(ps, s, splits, m, n, k, kchunk, A, lda, B, ldb, Cp, ldcp,    \
-                                                        alpha_re, alpha_im, b_re, b_im, part); break;                \
             }                                                                                                        \
         }                                                                                                            \
     }
@@ -602,30 +551,29 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     };
     // autotuned plan (the fixed-workspace entry point keeps the fixed rule, whose partials
     // it is sized for)
-    const int tmode = ws.ext || (F64 && !pipe) ? 0 : tune_mode();
+    const int tmode = ws.ext ? 0 : tune_mode();
     if (tmode > 0) {
         auto bucket = [](int x) { return x <= 2048 ? (x + 31) / 32 * 32 : (x + 1023) / 1024 * 1024; };
         char key[160];
         std::snprintf(key, sizeof(key), "gemm %s %c%c m=%d n=%d k=%d cu=%d", prec_tag, "NTC"[oa], "NTC"[ob],
                       bucket(m), bucket(n), bucket(k), cus);
         int a = 0, b = 0;
-        const int lo = F64 ? 12 : 0, hi = F64 ? 14 : 12;   // variants this precision has
-        if (tune_find(key, a, b) && a >= lo && a < hi && b >= 0 && b <= 6 && !(X32 && (a == 2 || a == 3 || a == 8))) {
+        if (tune_find(key, a, b) && has(a) && b >= 0 && b <= 6) {
             variant = a;
             occ = b;
         } else if (tmode == 2) {
             // candidates: every tile/map of the shape's kind, and for inner products every
             // split rule; timed into a scratch C (beta 0) so the caller's C is untouched
             std::vector<std::pair<int, int>> cand;
-            if (F64) {
-                for (int oc : {1, 2, 3})
-                    if (inner) cand.emplace_back(12, oc);
-                if (!inner) cand = {{12, 0}, {13, 0}};
+            if (!X32 && inner) {
+                for (int oc : {1, 2, 3, 6}) cand.emplace_back(12, oc);
+            } else if (!X32) {
+                cand = {{12, 0}, {13, 0}};
             } else if (inner) {
                 for (int v : {0, 1, 6, 7, 10, 11})
                     for (int oc : {1, 2, 3, 4, 6}) cand.emplace_back(v, oc);
             } else if (tall) {
-                for (int v : {3, 4, 0, 2, 8, 9}) cand.emplace_back(v, 0);
+                for (int v : {4, 0, 9}) cand.emplace_back(v, 0);
             } else {
                 for (int v : {0, 1, 5}) cand.emplace_back(v, 0);
             }
@@ -634,7 +582,6 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
             double best = 1e300;
             std::vector<std::pair<int, int>> seen;   // (variant, splits) already timed
             for (auto& c : cand) {
-                if (X32 && (c.first == 2 || c.first == 3 || c.first == 8)) continue;
                 const std::pair<int, int> vs(c.first, splits_of(c.first, c.second));
                 if (std::find(seen.begin(), seen.end(), vs) != seen.end()) continue;
                 seen.push_back(vs);
@@ -658,8 +605,8 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
 }  // namespace
 
 void gemm_reserve(GemmWorkspace& ws, int num_cu) {
-    // splits x tiles <= resident slots, so splits m n <= slots x BM x BN; the largest product
-    // of the split variants is 3 x 128 x 64 (c128: two doubles an element)
+    // splits x tiles <= slots, so splits m n <= slots x BM x BN; the largest product a CU is 6 slots
+    // of 64 x 64 (c128: two doubles an element)
     ws.part.reserve((size_t)3 * std::max(num_cu, 64) * 128 * 64 * 2 + 2);
 }
 

@@ -57,18 +57,16 @@ def run_solve(pw, ctx, ham, s, psi0_dev, precision):
 _PMC_FAMILY = {   # regular expressions over the kernel names of the committed traffic summary
     "eig_tridiag": r"apw::k_tridiag_(xcd|reg|rows|fused|lds)",
     # GEMMs: the path's updates are op(A) = N (tiled), its inner products op(A) = C (split-K)
-    # (template arguments: MFMA type, storage type, op(A), ...)
-    "zgemm_f64_tiled": r"apw::zgemm_kernel<double, double, 0, ",
-    "zgemm_f64_splitk": r"apw::zgemm_kernel<double, double, [12], ",
-    "cgemm_f32_tiled": r"apw::zgemm_kernel<float, float, 0, ", "cgemm_f32_splitk": r"apw::zgemm_kernel<float, float, [12], ",
-    "zgemm_x32_tiled": r"apw::zgemm_kernel<float, double, 0, ",
-    "zgemm_x32_splitk": r"apw::zgemm_kernel<float, double, [12], ",
+    # (zgemm_pipe<type, op(A), op(B)>; zgemm_kernel<op(A), op(B), ...> is the x32 form)
+    "zgemm_f64_tiled": r"apw::zgemm_pipe<double, 0, ", "zgemm_f64_splitk": r"apw::zgemm_pipe<double, [12], ",
+    "cgemm_f32_tiled": r"apw::zgemm_pipe<float, 0, ", "cgemm_f32_splitk": r"apw::zgemm_pipe<float, [12], ",
+    "zgemm_x32_tiled": r"apw::zgemm_kernel<0, ", "zgemm_x32_splitk": r"apw::zgemm_kernel<[12], ",
     "fft_x_veff_fused": r"apw::k_xreg<\w+, \d+, 0>|apw::k_xpass<\w+, 0>",
     "fft_y_bwd": r"apw::k_yreg<\w+, \d+, 1>|apw::k_ybwd", "fft_y_fwd": r"apw::k_yreg<\w+, \d+, -1>|apw::k_yfwd",
     "fft_z_bwd_scatter": r"apw::k_zreg<\w+, \d+, 1>|apw::k_zbwd",
     "fft_z_fwd_gather": r"apw::k_zreg<\w+, \d+, -1>|apw::k_zfwd",
     "eig_bisect": r"apw::k_bisect", "eig_invit": r"apw::k_invit",
-    "eig_backtransform": r"apw::k_(backtransform|wy_)|back-transform apw::(zgemm_kernel<double|splitk_reduce<double)",
+    "eig_backtransform": r"apw::k_(backtransform|wy_)|back-transform apw::(zgemm_pipe<double|splitk_reduce<double)",
     "chol_inv": r"apw::k_chol_inv",
 }
 # entries made of several dispatches per launch: the dispatches that occur once per launch
