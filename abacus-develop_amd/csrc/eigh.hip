@@ -971,30 +971,79 @@ __global__ __launch_bounds__(NTR) void k_tridiag_reg(const double2* __restrict__
     }
 }
 
+// x, the same in every lane, in scalar registers
+__device__ __forceinline__ double uniform_d(double x) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(x)));
+}
+__device__ __forceinline__ double2 uniform_d(double2 x) { return make_double2(uniform_d(x.x), uniform_d(x.y)); }
+
+// Sums over the 64 lanes of the 16 values (re, im) of eight columns, as wave_sums, taken in column
+// by column so that few are held at a time: 15 exchanges of halves within the 16-lane rows and
+// the row sum, against 16 x 4 steps one by one.  sum() holds the value of part (0: re, 1: im) bit 3
+// of the lane and column bits 0, 1, 2 = bits 2, 1, 0 of the lane.
+struct WaveSums8 {
+    double h[3], x;
+    template <int C>
+    __device__ __forceinline__ void add(double re, double im) {
+        // lane bits 3 .. 0 as constant masks: no register holds the lane for them
+        const bool b8 = __builtin_amdgcn_inverse_ballot_w64(0xFF00FF00FF00FF00ull);
+        const bool b4 = __builtin_amdgcn_inverse_ballot_w64(0xF0F0F0F0F0F0F0F0ull);
+        const bool b2 = __builtin_amdgcn_inverse_ballot_w64(0xCCCCCCCCCCCCCCCCull);
+        const bool b1 = __builtin_amdgcn_inverse_ballot_w64(0xAAAAAAAAAAAAAAAAull);
+        x = pair_merge<0x140>(re, im, b8);
+        if constexpr (C % 2 == 0) {
+            h[0] = x;
+        } else {
+            x = pair_merge<0x141>(h[0], x, b4);
+            if constexpr (C % 4 == 1) {
+                h[1] = x;
+            } else {
+                x = pair_merge<0x1B>(h[1], x, b2);
+                if constexpr (C == 3) h[2] = x;
+                else x = pair_merge<0xB1>(h[2], x, b1);
+            }
+        }
+    }
+    __device__ __forceinline__ double sum() const { return sum_rows_swapped(x); }
+};
+template <int I, int N, class F>
+__device__ __forceinline__ void unroll_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        unroll_for<I + 1, N>(f);
+    }
+}
+
 // Householder tridiagonalisation (lower) for large n (up to 64 * NW * CH rows): the own
 // columns stay in registers for the whole reduction, their rows split over the NW waves of
 // the workgroup (wave w, lane l holds rows 64 (w + NW ch) + l, ch < CH, of every own column),
 // so the trailing matrix never leaves the register files of the grid (at n = 1920 it is
 // 59 MB, more than all LDS together).  Same ownership and ring as k_tridiag_reg; each lane
-// polls only its own rows of p_k and of column k + 1.  The sums over rows v^H p and the
-// reflector norm are wave sums combined in LDS in a fixed order; the projections onto
-// v_{k+1} are summed over 16-lane rows only and the 4 NW row partials of a column combined
-// by wave 0.  Three workgroup barriers per column step.
-// LDS: y_k and v_k by row (2n), 4 NC NW projection partials, broadcast values, 2 NW sums.
+// polls only its own rows of q_k and of column k + 1.  Bound by the chain of one column step:
+// the exchange through memory, then sums over rows (wave sums combined in LDS in a fixed
+// order), the update of the own columns and the projection.  As in the one-XCD form the
+// projection is taken on the corrected column w, so that the norm, the square root, the
+// reciprocals and the reflector are formed while q = A^H w is on its way (n = 1920 to
+// column 1408: 11.7 -> 8.7 ms, 6.2 us a column; the sums of eight columns at once are 0.6 us of it).  Rows that the
+// reduction has passed are skipped wave by wave.  Three workgroup barriers per column step before
+// the publication, one after it.
+// LDS: y_k and v_k by row (2n), 16 NW projection partials, broadcast values, 2 NW sums.
 template <int CH, int NC, int NW>
 __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restrict__ A, int n, int ncol,
                                                          double2* __restrict__ V, double2* __restrict__ tau,
                                                          double* __restrict__ d, double* __restrict__ e,
                                                          double2* __restrict__ ring, unsigned* abort_flag,
                                                          int kstop, double2* __restrict__ sub) {
+    static_assert(NC == 8 && NW == 16, "projection sums: 16 values a wave, 16 waves");
     extern __shared__ __align__(16) unsigned char smem[];
     double2* yl = reinterpret_cast<double2*>(smem);   // y_k by row
     double2* vl = yl + n;                              // v_k by row
-    double2* pp = vl + n;                              // pp[(lc * NW + wave) * 4 + row]: partial projections
-    double2* bc = pp + 4 * NC * NW;                    // v_k, p_k, column k+1 at row k+1; alpha
-    double* red = reinterpret_cast<double*>(bc + 4);   // [NW] v^H p partials, [NW] norm partials
+    double2* bc = vl + n;                              // v_k, p_k, column k+1 at row k+1; alpha
+    double* pp = reinterpret_cast<double*>(bc + 4);    // pp[wave * 16 + lane]: partial projections
+    double* red = pp + 16 * NW;                        // [NW] v^H p partials, [NW] norm partials
     const int nwg = (int)gridDim.x, bid = (int)blockIdx.x;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     double2 cols[NC][CH];
 #pragma unroll
     for (int lc = 0; lc < NC; ++lc) {
@@ -1005,7 +1054,9 @@ __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restr
             cols[lc][ch] = (lc < ncol && c < n && i < n) ? A[(size_t)c * n + i] : make_double2(0.0, 0.0);
         }
     }
-    double2 v[CH], y[CH], w[CH];   // own rows of v_k, y_k, and the column / v_{k+1}
+    double2 v[CH], y[CH], w[CH];   // own rows of v_k, y_k, and the corrected column
+    double2 t, sc;                 // tau_k and 1 / (alpha - beta) of the current reflector
+    double beta;
     // the owning lane of row i stores x at row i into *dst
     auto own_put = [&](int i, const double2 (&x)[CH], double2* dst) {
         const int j = i >> 6;
@@ -1018,62 +1069,28 @@ __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restr
     // sum of the NW wave partials r[0..NW): one LDS read a lane and the same row tree in every
     // wave and every workgroup, so all of them get the same bits
     auto waves_sum = [&](const double* r) { return row_sum16((lane & 15) < NW ? r[lane & 15] : 0.0); };
-    // reflector of w on rows > k0 (as in k_tridiag_reg); one workgroup barrier
-    auto reflector = [&](int k0, double2& tv, double& beta) {
-        double s2 = 0;
-#pragma unroll
-        for (int ch = 0; ch < CH; ++ch) {
-            const int i = 64 * (wave + NW * ch) + lane;
-            if (i > k0 + 1 && i < n) s2 += w[ch].x * w[ch].x + w[ch].y * w[ch].y;
-        }
-        s2 = wave_sum(s2);
-        if (lane == 0) red[NW + wave] = s2;
-        own_put(k0 + 1, w, bc + 3);
-        __syncthreads();
-        const double xn2 = waves_sum(red + NW);
-        const double2 alpha = bc[3];
-        double2 sc;
-        if (xn2 == 0.0 && alpha.y == 0.0) {
-            tv = make_double2(0.0, 0.0);
-            beta = alpha.x;
-            sc = make_double2(0.0, 0.0);
-        } else {
-            const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xn2);
-            beta = alpha.x >= 0 ? -nrm : nrm;
-            const double rb = 1.0 / beta;
-            tv = make_double2((beta - alpha.x) * rb, -alpha.y * rb);
-            const double2 den = make_double2(alpha.x - beta, alpha.y);
-            const double rd = 1.0 / (den.x * den.x + den.y * den.y);
-            sc = make_double2(den.x * rd, -den.y * rd);
-        }
-#pragma unroll
-        for (int ch = 0; ch < CH; ++ch) {
-            const int i = 64 * (wave + NW * ch) + lane;
-            w[ch] = (i == k0 + 1) ? make_double2(1.0, 0.0)
-                                  : ((i > k0 + 1 && i < n) ? cmul(w[ch], sc) : make_double2(0.0, 0.0));
-        }
-    };
-    // as in k_tridiag_reg, with (y_c, v_c) read from LDS; one workgroup barrier before the
-    // per-column sums over the waves are published
+    // Publishes q_{k+1} = A_{k+1}^H w of the own columns c > k + 1 (and column k + 2 by its owner)
+    // into slot k + 1; update: after the rank-2 update of step k, with (y_c, v_c) from LDS.  w is
+    // zero on rows <= k + 1 and past n, v and y on rows <= k and past n, so the rows need no
+    // predicates: the update changes nothing there but row k + 1, which no later step reads.
+    // One workgroup barrier before the sums over the waves are published.
     auto update_and_project = [&](int k, bool update) {
         const __amdgpu_buffer_rsrc_t rs = ring_rsrc(ring + (size_t)(k + 1) * 2 * n, 2 * n);
-#pragma unroll
-        for (int lc = 0; lc < NC; ++lc) {
+        WaveSums8 sums;
+        unroll_for<0, NC>([&](auto lcc) {
+            constexpr int lc = decltype(lcc)::value;
             const int c = bid + lc * nwg;
+            double pr = 0, pi = 0;
             if (lc < ncol && c > k + 1 && c < n) {   // uniform over the workgroup
                 double2 yc = make_double2(0.0, 0.0), vc = make_double2(0.0, 0.0);
                 if (update) {
                     yc = yl[c];
                     vc = vl[c];
                 }
-                // every row, unpredicated: v_k and y_k are zero on rows <= k and past n, so
-                // the update changes nothing there but row k + 1, which no later step reads;
-                // v_{k+1} (in w) is zero on rows <= k + 1 and past n, so those rows add nothing
-                // to the projection
                 // a -= v_i conj(y_c) + y_i conj(v_c);  p += conj(a) w_i  (as FMA chains)
-                double pr = 0, pi = 0;
 #pragma unroll
                 for (int ch = 0; ch < CH; ++ch) {
+                    if (64 * (wave + NW * ch) + 63 <= k + 1) continue;   // rows done with (uniform over the wave)
                     double2 a = cols[lc][ch];
                     if (update) {
                         a.x = fma(-yc.x, v[ch].x, a.x);
@@ -1091,10 +1108,6 @@ __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restr
                     pi = fma(a.x, w[ch].y, pi);
                     pi = fma(-a.y, w[ch].x, pi);
                 }
-                // row sums only: the 4 rows of every wave go to LDS
-                pr = row_sum16(pr);
-                pi = row_sum16(pi);
-                if ((lane & 15) == 0) pp[(lc * NW + wave) * 4 + (lane >> 4)] = make_double2(pr, pi);
                 if (c == k + 2) {
 #pragma unroll
                     for (int ch = 0; ch < CH; ++ch) {
@@ -1103,59 +1116,79 @@ __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restr
                     }
                 }
             }
-        }
+            sums.add<lc>(pr, pi);
+        });
+        const double sum = sums.sum();
+        if (lane < 16) pp[wave * 16 + lane] = sum;
         __syncthreads();
-        // wave 0, lane 8 lc + g: partials g, g + 8, ... of column lc, then a tree over g
+        // wave 0, lane 16 g + j: partials of value j from waves g, g + 4, ..., then the sum over g
         if (wave == 0) {
-            // the lane id read afresh (volatile: not hoisted out of the column loop, where a
-            // long-lived per-lane column index was spilled to scratch)
-            int l;
-            asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-            const int lc = l >> 3, g = l & 7, c = bid + lc * nwg;
-            double re = 0, im = 0;
+            double x = 0;
 #pragma unroll
-            for (int q = g; q < 4 * NW; q += 8) {
-                const double2 t = pp[lc * NW * 4 + q];
-                re += t.x;
-                im += t.y;
-            }
-            re += dppm_d<0xB1>(re);
-            im += dppm_d<0xB1>(im);
-            re += dppm_d<0x4E>(re);
-            im += dppm_d<0x4E>(im);
-            re += dppm_d<0x141>(re);
-            im += dppm_d<0x141>(im);
-            if (g == 0 && lc < ncol && c > k + 1 && c < n) ring_put16(rs, c - (k + 2), make_double2(re, im));
+            for (int q = 0; q < NW / 4; ++q) x += pp[64 * q + lane];
+            x = sum_rows_swapped(x);
+            // re and im of a column are 8 lanes apart (l -> l ^ 8: row mirror, then half-row mirror)
+            const double im = dppm_d<0x141>(dppm_d<0x140>(x));
+            const int lc = ((lane >> 2) & 1) | (lane & 2) | ((lane << 2) & 4), c = bid + lc * nwg;
+            if (lane < 8 && lc < ncol && c > k + 1 && c < n) ring_put16(rs, c - (k + 2), make_double2(x, im));
+        }
+    };
+    // Reflector of w (rows > k0; alpha at row k0 + 1 in bc[3]): v, tau, beta, sc.  Off the chain:
+    // q is in flight.  One workgroup barrier.
+    auto reflector = [&](int k0, double dk) {
+        double s2 = 0;
+#pragma unroll
+        for (int ch = 0; ch < CH; ++ch) {
+            const int i = 64 * (wave + NW * ch) + lane;
+            if (i > k0 + 1 && i < n) s2 += w[ch].x * w[ch].x + w[ch].y * w[ch].y;
+        }
+        s2 = wave_sum(s2);
+        if (lane == 0) red[NW + wave] = s2;
+        __syncthreads();
+        const double xn2 = waves_sum(red + NW);
+        const double2 alpha = bc[3];
+        if (xn2 == 0.0 && alpha.y == 0.0) {
+            t = make_double2(0.0, 0.0);
+            beta = alpha.x;
+            sc = make_double2(0.0, 0.0);
+        } else {
+            const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xn2);
+            beta = alpha.x >= 0 ? -nrm : nrm;
+            const double rb = 1.0 / beta;
+            t = make_double2((beta - alpha.x) * rb, -alpha.y * rb);
+            const double2 den = make_double2(alpha.x - beta, alpha.y);
+            const double rd = 1.0 / (den.x * den.x + den.y * den.y);
+            sc = make_double2(den.x * rd, -den.y * rd);
+        }
+        t = uniform_d(t);   // 10 registers that the columns need
+        sc = uniform_d(sc);
+        beta = uniform_d(beta);
+#pragma unroll
+        for (int ch = 0; ch < CH; ++ch) {
+            const int i = 64 * (wave + NW * ch) + lane;
+            v[ch] = (i == k0 + 1) ? make_double2(1.0, 0.0)
+                                  : ((i > k0 + 1 && i < n) ? cmul(w[ch], sc) : make_double2(0.0, 0.0));
+            if (bid == 0 && i > k0 && i < n) V[(size_t)k0 * n + i] = v[ch];
+        }
+        if (bid == 0 && threadIdx.x == 0) {
+            tau[k0] = t;
+            d[k0] = dk;
+            e[k0] = beta;
         }
     };
     // first reflector from column 0 (rows 1 .. n-1)
-    double2 t;
-    double beta;
 #pragma unroll
     for (int ch = 0; ch < CH; ++ch) {
         const int i = 64 * (wave + NW * ch) + lane;
         w[ch] = (i >= 1 && i < n) ? A[i] : make_double2(0.0, 0.0);
+        v[ch] = y[ch] = make_double2(0.0, 0.0);
     }
-    reflector(0, t, beta);
-    if (bid == 0) {
-#pragma unroll
-        for (int ch = 0; ch < CH; ++ch) {
-            const int i = 64 * (wave + NW * ch) + lane;
-            if (i >= 1 && i < n) V[i] = w[ch];
-        }
-        if (threadIdx.x == 0) {
-            tau[0] = t;
-            d[0] = A[0].x;
-            e[0] = beta;
-        }
-    }
+    own_put(1, w, bc + 3);
     update_and_project(-1, false);
-#pragma unroll
-    for (int ch = 0; ch < CH; ++ch) v[ch] = w[ch];
+    reflector(0, A[0].x);
     for (int k = 0; k < n - 1; ++k) {
-        const int m = n - k - 1;
         const __amdgpu_buffer_rsrc_t rs = ring_rsrc(ring + (size_t)k * 2 * n, 2 * n);
-        // ---- own rows of p_k (-> y) and of column k+1 (-> w) ----
+        // ---- own rows of q_k (-> y) and of column k+1 (-> w) ----
 #pragma unroll
         for (int ch = 0; ch < CH; ++ch) {
             y[ch] = make_double2(0.0, 0.0);
@@ -1203,10 +1236,13 @@ __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restr
                 __builtin_amdgcn_s_sleep(1);
             }
         }
-        // ---- mu = v^H p over the workgroup; y = tau p - (|tau|^2 mu / 2) v ----
+        // ---- p = sc (q - beta column); mu = v^H p over the workgroup; y = tau p - (|tau|^2 mu / 2) v ----
         double mr = 0;
 #pragma unroll
-        for (int ch = 0; ch < CH; ++ch) mr += cconjmul(v[ch], y[ch]).x;
+        for (int ch = 0; ch < CH; ++ch) {
+            y[ch] = cmul(sc, make_double2(fma(-beta, w[ch].x, y[ch].x), fma(-beta, w[ch].y, y[ch].y)));
+            mr += cconjmul(v[ch], y[ch]).x;
+        }
         mr = wave_sum(mr);
         if (lane == 0) red[wave] = mr;
         own_put(k + 1, v, bc + 0);
@@ -1237,7 +1273,7 @@ __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restr
             const double2 a2 = cconjmul(y0, v0);
             dk1 = bc[2].x - (a1.x + a2.x);
         }
-        if (m >= 2) {
+        if (k < n - 2) {
             // y_k and v_k by row, for the (y_c, v_c) of the own columns' updates
 #pragma unroll
             for (int ch = 0; ch < CH; ++ch) {
@@ -1248,25 +1284,13 @@ __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restr
                 }
             }
             if (k + 1 == kstop) break;   // y_k, v_k in yl, vl; column k+1 in w
-            double2 tn;
-            double bn;
-            reflector(k + 1, tn, bn);
-            if (bid == 0) {
+            own_put(k + 2, w, bc + 3);
 #pragma unroll
-                for (int ch = 0; ch < CH; ++ch) {
-                    const int i = 64 * (wave + NW * ch) + lane;
-                    if (i >= k + 2 && i < n) V[(size_t)(k + 1) * n + i] = w[ch];
-                }
-                if (threadIdx.x == 0) {
-                    tau[k + 1] = tn;
-                    d[k + 1] = dk1;
-                    e[k + 1] = bn;
-                }
-            }
+            for (int ch = 0; ch < CH; ++ch)
+                if (64 * (wave + NW * ch) + lane <= k + 1) w[ch] = make_double2(0.0, 0.0);
+            __syncthreads();
             update_and_project(k, true);
-#pragma unroll
-            for (int ch = 0; ch < CH; ++ch) v[ch] = w[ch];
-            t = tn;
+            reflector(k + 1, dk1);
         } else if (bid == 0 && threadIdx.x == 0) {
             d[k + 1] = dk1;
         }
@@ -2438,8 +2462,7 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
             auto run_rows = [&](int wg) {
                 int ncol_r = (n + wg - 1) / wg;
                 constexpr int nw = 16;
-                const size_t lds = (size_t)2 * n * sizeof(double2) + (size_t)(4 * 8 * nw + 4) * sizeof(double2) +
-                                   (size_t)2 * nw * sizeof(double);
+                const size_t lds = (size_t)(2 * n + 4) * sizeof(double2) + (size_t)(16 * nw + 2 * nw) * sizeof(double);
                 const void* fn = reinterpret_cast<const void*>(k_tridiag_rows<2, 8, nw>);
                 APW_CHECK(ncol_r <= 8 && n <= 64 * 32, "heevx: row-split form cannot take n=%d on %d workgroups", n, wg);
                 APW_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
