@@ -1024,10 +1024,10 @@ __device__ __forceinline__ void unroll_for(F&& f) {
 // the exchange through memory, then sums over rows (wave sums combined in LDS in a fixed
 // order), the update of the own columns and the projection.  As in the one-XCD form the
 // projection is taken on the corrected column w, so that the norm, the square root, the
-// reciprocals and the reflector are formed while q = A^H w is on its way (n = 1920 to
-// column 1408: 11.7 -> 8.7 ms, 6.2 us a column; the sums of eight columns at once are 0.6 us of it).  Rows that the
-// reduction has passed are skipped wave by wave.  Three workgroup barriers per column step before
-// the publication, one after it.
+// reciprocals and the reflector are formed while q = A^H w is on its way; the projections of
+// all own columns are summed over lanes together, and rows that the reduction has passed are
+// skipped wave by wave (n = 1920 to column 1408: 11.7 -> 8.7 ms, 6.2 us a column).  Three
+// workgroup barriers per column step before the publication, one after it.
 // LDS: y_k and v_k by row (2n), 16 NW projection partials, broadcast values, 2 NW sums.
 template <int CH, int NC, int NW>
 __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restrict__ A, int n, int ncol,
