@@ -395,7 +395,15 @@ void launch_pipe(ProfScope& ps, hipStream_t s, int map, int splits, int M, int N
                  int lda, const R* B, int ldb, R* C, int ldc, double ar, double ai, double br, double bi, R* part) {
     using c_t = typename ZpType<R>::c_t;
     const int tm = (M + ZP_BM - 1) / ZP_BM, tn = (N + ZP_BN - 1) / ZP_BN;
-    const dim3 grid = map == 1 ? dim3((unsigned)(((tm + 7) / 8) * 8 * tn), 1, splits) : dim3(tm, tn, splits);
+    // the balanced order of map 2 up to four n-tiles (us a product with its reduction, map 0 -> 2:
+    // 640 x 160 x 51627 615 -> 542, 577 x 97 424 -> 404, 160 x 160 199 -> 176, 1024 x 256 x 228487
+    // 5540 -> 5405); with eight the narrow one matters little and m-major shares more of A
+    // (480 x 480 x 228487: 5676, map 2 5811)
+    if (map == 0 && splits > 1 && N <= 4 * ZP_BN) map = 2;
+    const int narrow = N % ZP_BN ? splits * tm : 0, wide = splits * tm * (N / ZP_BN);
+    const dim3 grid = map == 2   ? dim3((unsigned)(8 * (zp_share(wide) + zp_share(narrow))))
+                      : map == 1 ? dim3((unsigned)(((tm + 7) / 8) * 8 * tn), 1, splits)
+                                 : dim3(tm, tn, splits);
     APW_PLAUNCH(ps, (zgemm_pipe<R, TA, TB>), grid, dim3(ZP_NT), 0, s, M, N, K, kchunk, map,
                 reinterpret_cast<const c_t*>(A), lda, reinterpret_cast<const c_t*>(B), ldb,
                 reinterpret_cast<c_t*>(C), ldc, ar, ai, br, bi, reinterpret_cast<c_t*>(part));
@@ -444,6 +452,13 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
         if (occ <= 0) return 1;
         const long tiles = tiles_of(VBM[v], VBN[v]), slots = (long)occ * cus;
         int sp = tiles < slots ? (int)(slots / tiles) : 1;
+        if (!X32) {   // the shares of an XCD in its resident slots too
+            const int tm = (m + ZP_BM - 1) / ZP_BM;
+            auto share = [&] {
+                return zp_share(sp * tm * (n / ZP_BN)) + (n % ZP_BN ? zp_share(sp * tm) : 0);
+            };
+            while (sp > 1 && (long)share() * 8 > slots) --sp;
+        }
         sp = std::max(1, std::min(std::min(sp, std::max(1, k / 64)), 256));
         int kc = (k + sp - 1) / sp;
         kc = (kc + BKMAX - 1) / BKMAX * BKMAX;

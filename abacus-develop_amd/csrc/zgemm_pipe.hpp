@@ -245,7 +245,12 @@ __device__ __forceinline__ void zp_tile(int M, int N, const typename ZpType<R>::
 // op codes: 0 = N, 1 = T, 2 = C.  map 0: grid (m-tiles, n-tiles,
 // splits); map 1 (1-D grid in x padded to a multiple of 8 m-tiles): workgroup L runs on
 // XCD L % 8, so each XCD takes whole m-tiles and walks their n-tiles back to back, and the
-// rows of A that they share stay in its L2.
+// rows of A that they share stay in its L2.  map 2 (k split so that all workgroups are resident,
+// 1-D grid of 8 (zp_share(wide) + zp_share(narrow))): each XCD takes an eighth of the splits, all
+// full-width tiles before those of the last, narrower n-tile, so that the workgroups that meet
+// on a CU (one every num_cu / 8 of an XCD) are a like mix of both on every CU; with m-major order
+// some CUs got the wide ones only.
+__host__ __device__ inline int zp_share(int tiles) { return (tiles + 7) / 8; }
 template <class R, int TA, int TB>
 __global__ __launch_bounds__(ZP_NT, ZP_OCC) void zgemm_pipe(int M, int N, int K, int kchunk, int map,
                                                             const typename ZpType<R>::c_t* __restrict__ A, int lda,
@@ -262,6 +267,24 @@ __global__ __launch_bounds__(ZP_NT, ZP_OCC) void zgemm_pipe(int M, int N, int K,
         bm = (L % 8) + 8 * (L / (8 * ntn));
         bn = (L / 8) % ntn;
         if (bm >= (M + ZP_BM - 1) / ZP_BM) return;
+    }
+    if (map == 2) {
+        const int tmt = (M + ZP_BM - 1) / ZP_BM, nw = N / ZP_BN, splits = (K + kchunk - 1) / kchunk;
+        const int wide = splits * tmt * nw, narrow = N % ZP_BN ? splits * tmt : 0;
+        const int x = blockIdx.x % 8, j = blockIdx.x / 8;
+        int g;
+        if (j < zp_share(wide)) {
+            g = x * zp_share(wide) + j;
+            if (g >= wide) return;
+            bn = g % nw;
+            g /= nw;
+        } else {
+            g = x * zp_share(narrow) + j - zp_share(wide);
+            if (g >= narrow) return;
+            bn = nw;
+        }
+        bm = g % tmt;
+        sp = g / tmt;
     }
     const int m0 = bm * ZP_BM, n0 = bn * ZP_BN;
     const int kbeg = sp * kchunk, kend = min(K, kbeg + kchunk);
