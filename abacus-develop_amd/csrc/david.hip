@@ -35,6 +35,21 @@ namespace {
 
 int gsz(size_t n) { return (int)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 8192)); }
 
+// What the host reads in an iteration, stored by one workgroup into pinned host memory (a copy of
+// each took 4 to 5 us on the stream): the breakdown words, which it clears, the eigensolver's, the
+// eigenvalues and nres residual norms.
+__global__ void k_fetch(int* __restrict__ status, const unsigned* __restrict__ bar, const double* __restrict__ eig,
+                        int nband, const double* __restrict__ resid, int nres, int* __restrict__ h_status,
+                        unsigned* __restrict__ h_bar, double* __restrict__ h_vals) {
+    if (threadIdx.x < 2) {
+        h_status[threadIdx.x] = status[threadIdx.x];
+        status[threadIdx.x] = 0;
+        h_bar[threadIdx.x] = bar ? bar[threadIdx.x] : 0u;
+    }
+    for (int i = threadIdx.x; i < nband; i += blockDim.x) h_vals[i] = eig[i];
+    for (int i = threadIdx.x; i < nres; i += blockDim.x) h_vals[nband + i] = resid[i];
+}
+
 // c128 <-> c64 column blocks (precision=single callers: c64 psi and callbacks)
 __global__ void k_cols_narrow(int rows, int ncols, const double2* __restrict__ src, int lds, float2* __restrict__ dst,
                               int ldd) {
@@ -138,7 +153,7 @@ struct David {
     apw_ctx* ctx = nullptr;
     int nband = 0, dim = 0, ndim = 0, nbx = 0;
     DevBuf<double> pre, basis, hp, sp, hcc, vcc, eig, tmp, vc, lmat, resid;
-    DevBuf<int> unconv_d, need_d, status;
+    DevBuf<int> lists_d, status;   // lists_d: the unconverged bands, then a flag for each band
     EigWorkspace ews;
     GemmWorkspace& gws() { return ctx->gws; }   // shared by the context: sized once
 
@@ -157,7 +172,7 @@ struct David {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> hev;
     // pinned host block: [status 2 int][barrier words 2 uint][eig nband][resid nband][unconv nband int]
     // [need nband int]
-    unsigned char* hbuf = nullptr;
+    unsigned char *hbuf = nullptr, *hdev = nullptr;   // hdev: the same memory for kernels
     size_t hbuf_bytes() const { return 16 + (size_t)2 * nband * sizeof(double) + (size_t)2 * nband * sizeof(int); }
     int* h_status() { return reinterpret_cast<int*>(hbuf); }
     unsigned* h_bar() { return reinterpret_cast<unsigned*>(hbuf + 8); }
@@ -196,13 +211,13 @@ struct David {
         vc.reserve((size_t)2 * nbx * nband);
         lmat.reserve((size_t)2 * nbx * nband);
         resid.reserve(nbx);
-        unconv_d.reserve(nband);
-        need_d.reserve(nband);
+        lists_d.reserve((size_t)2 * nband);
         status.reserve(4);
         heevx_reserve(ews, nbx, nband);
         gemm_reserve(ctx->gws, ctx->num_cu);
         // pinned host words of the per-iteration reads (pageable copies go through staging)
         APW_HIP(hipHostMalloc(reinterpret_cast<void**>(&hbuf), hbuf_bytes(), hipHostMallocDefault));
+        APW_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&hdev), hbuf, 0));
         zero(st(), (size_t)2 * nbx * nbx, vcc.get());
         zero(st(), (size_t)2 * nbx * nbx, hcc.get());
         APW_LAUNCH_CHECK();
@@ -281,8 +296,6 @@ struct David {
     // block classical Gram-Schmidt with Pythagorean norms (SchmidtOrth, diago_david.cpp:950-1075),
     // in blocks of at most CHOL_MAX columns, each against everything before it.
     void orthonormalize(int c0, int nc) {
-        zero(st(), (size_t)2, reinterpret_cast<double*>(status.get()));
-        APW_LAUNCH_CHECK();
         // equal blocks rounded up to whole 32-column GEMM tiles (two blocks of 80 left 16
         // columns of every third tile idle in the block's products; 96 + 64 fill them)
         const int nblk = (nc + CHOL_MAX - 1) / CHOL_MAX;
@@ -315,11 +328,10 @@ struct David {
     // the breakdown and time-out words, the eigenvalues and (nres > 0) residual norms in one
     // host round trip; throws on a breakdown or a time-out
     void fetch_iteration(int nres) {
-        APW_HIP(hipMemcpyAsync(h_status(), status.get(), 2 * sizeof(int), hipMemcpyDeviceToHost, st()));
-        h_bar()[0] = h_bar()[1] = 0;
-        if (ews.bar.get()) APW_HIP(hipMemcpyAsync(h_bar(), ews.bar.get(), 2 * sizeof(unsigned), hipMemcpyDeviceToHost, st()));
-        APW_HIP(hipMemcpyAsync(h_eig(), eig.get(), nband * sizeof(double), hipMemcpyDeviceToHost, st()));
-        if (nres > 0) APW_HIP(hipMemcpyAsync(h_res(), resid.get(), nres * sizeof(double), hipMemcpyDeviceToHost, st()));
+        hipLaunchKernelGGL(k_fetch, dim3(1), dim3(256), 0, st(), status.get(), ews.bar.get(), eig.get(), nband,
+                           resid.get(), nres, reinterpret_cast<int*>(hdev), reinterpret_cast<unsigned*>(hdev + 8),
+                           reinterpret_cast<double*>(hdev + 16));
+        APW_LAUNCH_CHECK();
         APW_HIP(hipStreamSynchronize(st()));
         check_words(h_status(), h_bar());
     }
@@ -350,19 +362,18 @@ struct David {
         ews.single_max = ctx->eig_single_max;
         heevx_values(st(), ews, ctx->num_cu, nbase, nbx, hcc.get(), nband, eig.get(), &ctx->prof);
     }
+    // The unconverged bands and a flag for each band, in one copy.  (The pinned lists are rewritten
+    // only after the next fetch_iteration has synchronised the stream: this copy has completed.)
+    void send_lists(const std::vector<int>& unconv, int notconv) {
+        std::copy(unconv.begin(), unconv.begin() + notconv, h_unconv());
+        std::fill(h_need(), h_need() + nband, 0);
+        for (int m = 0; m < notconv; ++m) h_need()[unconv[m]] = 1;
+        APW_HIP(hipMemcpyAsync(lists_d.get(), h_unconv(), (size_t)2 * nband * sizeof(int), hipMemcpyHostToDevice, st()));
+    }
     // all eigenvectors (every column of vcc is read: psi = basis vcc and refresh), or only those
     // of the unconverged bands (cal_grad reads vcc[:, unconv] alone)
-    void solve_vectors(int nbase, bool all, const std::vector<int>& unconv, int notconv) {
-        const int* need = nullptr;
-        if (!all) {
-            // the pinned need block is rewritten only after the next fetch_iteration has
-            // synchronised the stream, so this copy has completed by then
-            int* hn = h_need();
-            std::fill(hn, hn + nband, 0);
-            for (int m = 0; m < notconv; ++m) hn[unconv[m]] = 1;
-            APW_HIP(hipMemcpyAsync(need_d.get(), hn, nband * sizeof(int), hipMemcpyHostToDevice, st()));
-            need = need_d.get();
-        }
+    void solve_vectors(int nbase, bool all, int notconv) {
+        const int* need = all ? nullptr : lists_d.get() + nband;
         heevx_vectors(st(), ews, gws(), ctx->num_cu, nbase, nband, eig.get(), vcc.get(), nbx, need, all ? nband : notconv,
                       &ctx->prof);
     }
@@ -380,6 +391,7 @@ struct David {
         std::vector<int> unconv(nband);
         for (int m = 0; m < nband; ++m) unconv[m] = m;
         int notconv = nband;
+        zero(st(), (size_t)1, reinterpret_cast<double*>(status.get()));   // k_fetch leaves it so
         // initial orthonormalisation of the start vectors (:186-228)
         copy_cols(st(), dim, nband,
                   reinterpret_cast<const double2*>(psi), ldpsi, reinterpret_cast<double2*>(basis.get()), dim);
@@ -391,21 +403,18 @@ struct David {
         solve_subspace(nbase);
         fetch_iteration(0);
         std::copy(h_eig(), h_eig() + nband, eig_host);
+        send_lists(unconv, notconv);
         int it = 0;
         while (true) {
             ++it;
             // ---- cal_grad (:359-611) ----
-            // (the pinned unconv block is not rewritten before the stream has consumed it: the
-            // next write follows the synchronisation of fetch_iteration below)
-            std::copy(unconv.begin(), unconv.begin() + notconv, h_unconv());
-            APW_HIP(hipMemcpyAsync(unconv_d.get(), h_unconv(), notconv * sizeof(int), hipMemcpyHostToDevice, st()));
             double2* vcp = reinterpret_cast<double2*>(vc.get());
             gather_cols(st(), nbase, notconv,
-                        reinterpret_cast<const double2*>(vcc.get()), nbx, unconv_d.get(), vcp);
+                        reinterpret_cast<const double2*>(vcc.get()), nbx, lists_d.get(), vcp);
             double* NB = Bd(basis.get(), nbase);
             gemm_sub('N', 'N', dim, notconv, nbase, 1.0, hp.get(), dim, vc.get(), nbase, 0.0, NB, dim);
             hipLaunchKernelGGL(k_scale_vc, dim3(gsz((size_t)nbase * notconv)), dim3(256), 0, st(), nbase, notconv, vcp,
-                               eig.get(), unconv_d.get());
+                               eig.get(), lists_d.get());
             gemm_sub('N', 'N', dim, notconv, nbase, 1.0, S(), dim, vc.get(), nbase, 1.0, NB, dim);
             if (switch_thr > 0) {
                 hipLaunchKernelGGL(k_colres2, dim3(notconv), dim3(CR_NT), 0, st(), dim,
@@ -434,8 +443,10 @@ struct David {
                 eig_host[m] = ehost[m];
             }
             const bool leave_mixed = switch_thr > 0 && (rmax < switch_thr || notconv == 0);
-            const bool full = !notconv || nbase + notconv > nbx || it == maxiter || leave_mixed;
-            solve_vectors(nbase, full, unconv, notconv);
+            const bool done = !notconv || it == maxiter || leave_mixed;
+            const bool full = done || nbase + notconv > nbx;
+            if (!done) send_lists(unconv, notconv);
+            solve_vectors(nbase, full, notconv);
             if (full) {
                 // psi = basis vcc (:292-306)
                 gemm('N', 'N', dim, nband, nbase, 1.0, basis.get(), dim, vcc.get(), nbx, 0.0, psi, ldpsi);
@@ -444,7 +455,7 @@ struct David {
                               ldpsi, nband, reinterpret_cast<double2*>(psi), ldpsi);
                     APW_LAUNCH_CHECK();
                 }
-                if (!notconv || it == maxiter || leave_mixed) {
+                if (done) {
                     // residual norms ||H psi_m - e_m psi_m|| of the returned vectors, from the
                     // subspace (hpsi vcc - e psi): one GEMM, no extra H application
                     gemm('N', 'N', dim, nband, nbase, 1.0, hp.get(), dim, vcc.get(), nbx, 0.0, tmp.get(), dim);
@@ -452,11 +463,9 @@ struct David {
                                        reinterpret_cast<const double2*>(tmp.get()), dim,
                                        reinterpret_cast<const double2*>(psi), ldpsi, eig.get(), resid.get());
                     APW_LAUNCH_CHECK();
-                    std::vector<double> r2(nband);
-                    APW_HIP(hipMemcpyAsync(r2.data(), resid.get(), nband * sizeof(double), hipMemcpyDeviceToHost, st()));
-                    APW_HIP(hipStreamSynchronize(st()));
+                    fetch_iteration(nband);
                     last_resid = 0;
-                    for (double v : r2) last_resid = std::max(last_resid, std::sqrt(v));
+                    for (int m = 0; m < nband; ++m) last_resid = std::max(last_resid, std::sqrt(h_res()[m]));
                     break;
                 }
                 // refresh (:797-934)
