@@ -400,6 +400,7 @@ void launch_pipe(ProfScope& ps, hipStream_t s, int map, int splits, int M, int N
     // 5540 -> 5405); with eight the narrow one matters little and m-major shares more of A
     // (480 x 480 x 228487: 5676, map 2 5811)
     if (map == 0 && splits > 1 && N <= 4 * ZP_BN) map = 2;
+    if (map == 0 && tn > 65535) map = 1;   // past the grid's second dimension
     const int narrow = N % ZP_BN ? splits * tm : 0, wide = splits * tm * (N / ZP_BN);
     const dim3 grid = map == 2   ? dim3((unsigned)(8 * (zp_share(wide) + zp_share(narrow))))
                       : map == 1 ? dim3((unsigned)(((tm + 7) / 8) * 8 * tn), 1, splits)

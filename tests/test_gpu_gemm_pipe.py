@@ -107,6 +107,11 @@ def test_half_aligned(torch, tuner, ops, m, n, k, single):
     _check(torch, tuner, ops, m, n, k, pad=1, half=True, single=single)
 
 
+def test_many_columns(torch, tuner):
+    """More n-tiles than a grid's second dimension holds."""
+    _check(torch, tuner, "NN", 2, 65535 * 64 + 70, 3, pad=0)
+
+
 @pytest.mark.parametrize("m,n,k", [(541, 13, 7106), (64, 64, 72), (300, 100, 40000)])
 @pytest.mark.parametrize("single", [False, True])
 def test_same_bits(torch, tuner, m, n, k, single):
