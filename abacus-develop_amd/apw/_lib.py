@@ -56,6 +56,7 @@ PROTOTYPES = {
     "apw_ctx_stream": (_vp, [_vp]),
     "apw_ctx_set_profiling": (_i, [_vp, _i]),
     "apw_ctx_set_eig_single_wg": (_i, [_vp, _i]),
+    "apw_ctx_fill_workspaces": (_i, [_vp, _d]),
     "apw_ctx_profile_count": (_i, [_vp]),
     "apw_ctx_profile_entry": (_i, [_vp, _i, C.c_char_p, _i, C.POINTER(C.c_longlong), C.POINTER(_d), C.POINTER(_d),
                                    C.POINTER(_d)]),

@@ -68,6 +68,10 @@ class Context:
         of the reductions: concurrent small solves on several contexts)."""
         check(self.lib.apw_ctx_set_eig_single_wg(self.handle, int(nmax)))
 
+    def fill_workspaces(self, value: float):
+        """Stores value in the context's work arrays, whose contents no call may depend on."""
+        check(self.lib.apw_ctx_fill_workspaces(self.handle, float(value)))
+
     def set_profiling(self, on: bool):
         check(self.lib.apw_ctx_set_profiling(self.handle, int(on)))
 

@@ -1,4 +1,5 @@
 // Context (device + stream), error reporting and the gemm_op mirror of the C ABI.
+#include <algorithm>
 #include <cstring>
 
 #include "apw_internal.hpp"
@@ -110,6 +111,12 @@ ProfScope::~ProfScope() {
     if (hipEventRecord(b, s) == hipSuccess) e->pending.emplace_back(a, b);
 }
 
+namespace {
+__global__ void k_fill(size_t n, double value, double* __restrict__ x) {
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) x[i] = value;
+}
+}  // namespace
+
 }  // namespace apw
 
 using apw::guarded;
@@ -186,6 +193,24 @@ int apw_ctx_set_eig_single_wg(apw_ctx* ctx, int nmax) {
     return guarded([&] {
         APW_CHECK(ctx && nmax >= 0, "apw_ctx_set_eig_single_wg: null ctx or negative size");
         ctx->eig_single_max = nmax;
+        return (int)APW_OK;
+    });
+}
+
+int apw_ctx_fill_workspaces(apw_ctx* ctx, double value) {
+    return guarded([&] {
+        APW_CHECK(ctx, "apw_ctx_fill_workspaces: null ctx");
+        apw::DeviceGuard g(ctx->device);
+        apw::EigWorkspace& e = ctx->ews;
+        apw::GenWorkspace& q = ctx->gen;
+        for (apw::DevBuf<double>* b : {&ctx->scratch, &ctx->gws.part, &ctx->gws.tune_c, &e.a, &e.v, &e.tau, &e.d, &e.e,
+                                       &e.ring, &e.sub, &e.z, &e.zc, &e.wy, &q.a, &q.r, &q.t, &q.x, &q.c, &q.t2, &q.y}) {
+            if (!b->get()) continue;
+            hipLaunchKernelGGL(apw::k_fill, dim3((unsigned)std::min<size_t>(4096, (b->n + 255) / 256)), dim3(256), 0,
+                               ctx->stream, b->n, value, b->get());
+            APW_LAUNCH_CHECK();
+        }
+        APW_HIP(hipStreamSynchronize(ctx->stream));
         return (int)APW_OK;
     });
 }

@@ -492,7 +492,8 @@ __global__ __launch_bounds__(NT) void k_tridiag_xcd(const double2* __restrict__ 
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int i = lane + 64 * r;
-            cols[lc][r] = (c < n && i < n) ? A[(size_t)c * n + i] : make_double2(0.0, 0.0);
+            // row 0 is in no update or projection, and the hand-over does not write it
+            cols[lc][r] = (c < n && i > 0 && i < n) ? A[(size_t)c * n + i] : make_double2(0.0, 0.0);
         }
     }
     double2 t, sc;

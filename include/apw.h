@@ -63,6 +63,11 @@ void* apw_ctx_stream(apw_ctx* ctx);
  * many small solves on different streams (batched k-points or cells) run at the same time;
  * 0 (the default) never does.  The eigenpairs are those of the cooperative form. */
 int apw_ctx_set_eig_single_wg(apw_ctx* ctx, int nmax);
+
+/* No counterpart in the reference.  Stores value in every element of the context's floating-point
+ * work arrays, as far as they have been allocated: no call may depend on what they hold, which
+ * the unit tests check with NaN. */
+int apw_ctx_fill_workspaces(apw_ctx* ctx, double value);
 /* Kernel profiler (no counterpart in the reference, whose ModuleBase::timer is host-side,
  * timer.cpp:71-130): when on, the library's kernels are bracketed by HIP events on the
  * context stream and accumulated per kernel name with their algorithmic HBM bytes and
