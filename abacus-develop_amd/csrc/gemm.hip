@@ -486,7 +486,7 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     const char* prec_tag = X32 ? "x32" : (std::is_same<R, double>::value ? "f64" : "f32");
     auto need_of = [&](int v, int oc) {
         const int sp = splits_of(v, oc);
-        return sp > 1 ? (size_t)sp * m * n * 2 * sizeof(S) / sizeof(double) + 2 : (size_t)0;
+        return sp > 1 ? (size_t)sp * m * n * 2 * sizeof(S) / sizeof(double) : (size_t)0;   // doubles
     };
     // runs a plan: C = alpha op(A) op(B) + beta C through the split partials when it splits
     auto run = [&](int v, int oc, S* Cp, int ldcp, double b_re, double b_im, Prof* pf) {

@@ -63,3 +63,25 @@ def test_zgemm_noalloc_matches_zgemm(torch, ta, tb):
         bound = 8 * k * np.finfo(float).eps * (np.abs(op_a) @ np.abs(B.T)).max() * abs(alpha) + 1e-12
         assert np.abs(got_new - want).max() < bound
     ctx.close()
+
+
+# products whose splits fill every resident workgroup with whole 64 x 64 tiles: their partials take
+# the fixed array to its last element
+@pytest.mark.parametrize("m,n,k", [(128, 128, 12288), (256, 256, 15360), (64, 192, 16384)])
+def test_zgemm_noalloc_fills_its_array(torch, m, n, k):
+    from apw import pw
+    ctx = pw.Context(0)
+    print(f"zgemm_noalloc CN m={m} n={n} k={k}", flush=True)
+    A = torch.randn((m, k), dtype=torch.complex128, device="cuda")
+    B = torch.randn((n, k), dtype=torch.complex128, device="cuda")
+    c_ref = torch.zeros((n, m), dtype=torch.complex128, device="cuda")
+    c_new = torch.zeros((n, m), dtype=torch.complex128, device="cuda")
+    _call(ctx, ctx.lib.apw_zgemm, "C", "N", m, n, k, 1 + 0j, A, k, B, k, 0j, c_ref, m)
+    _call(ctx, ctx.lib.apw_zgemm_noalloc, "C", "N", m, n, k, 1 + 0j, A, k, B, k, 0j, c_new, m)
+    got = c_new.cpu().numpy()
+    assert np.array_equal(c_ref.cpu().numpy(), got)
+    a, b = A.cpu().numpy(), B.cpu().numpy()
+    want = (a.conj() @ b.T).T
+    bound = 8 * k * np.finfo(float).eps * (np.abs(a) @ np.abs(b).T).max()
+    assert np.abs(got - want).max() < bound
+    ctx.close()
