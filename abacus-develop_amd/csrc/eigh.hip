@@ -1329,9 +1329,10 @@ __global__ __launch_bounds__(NW * 64) void k_tridiag_rows(const double2* __restr
 // Sturm count: number of eigenvalues of T below x, the sign changes in the characteristic
 // polynomials of the leading blocks, p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2} (division-free;
 // the ratio q_i = p_i / p_{i-1} of the LAPACK form is never formed).  An exact zero takes the sign
-// of its zero: between neighbours of opposite sign (p_{i+1} = -e^2 p_{i-1}) it adds one change
-// either way, and as the last value it puts an eigenvalue equal to x on either side.  p and
-// p_{i-1} are rescaled by a power of two every 8 steps (the recurrence is homogeneous).
+// of its zero: its neighbours have opposite signs (p_{i+1} = -e^2 p_{i-1}, so e must not be zero or
+// so small that this underflows: sturm_split takes such T), and it adds one change either way;
+// as the last value it puts an eigenvalue equal to x on either side.  p and p_{i-1} are rescaled
+// by a power of two every 8 steps (the recurrence is homogeneous).
 // de[i] = (d_i, -e_{i-1}^2) in LDS, with 16 more that are read and not used; every lane of a
 // wave reads the same address.
 // Bound by the issue of one wave a SIMD: four instructions a step -- the recurrence, and the sign
@@ -1377,6 +1378,22 @@ __device__ int sturm(const double2* de, int n, double x) {
     return c;
 }
 
+// The same count for a T that decouples: where e is zero, a p of exactly zero (x equal to an
+// eigenvalue of the blocks so far) would leave nothing but zeros, and the count would miss or
+// add eigenvalues of the blocks that follow.  The ratio form has no such state: q_i = d_i - x -
+// e_{i-1}^2 / q_{i-1}, with a q within pivmin of zero counted as negative (LAPACK's rule).  The
+// division makes it several times slower; a dense matrix's T does not come here.
+__device__ int sturm_split(const double2* de, int n, double x, double pivmin) {
+    int c = 0;
+    double q = 1.0;   // de[0].y is zero
+    for (int i = 0; i < n; ++i) {
+        q = (de[i].x - x) + de[i].y / q;
+        if (fabs(q) <= pivmin) q = -pivmin;
+        c += q < 0.0;
+    }
+    return c;
+}
+
 // Multisection: one wave per eigenvalue index j; each step the 64 lanes evaluate the Sturm
 // count at 64 interior points of [lo, hi] and the wave keeps the sub-interval holding the
 // j-th eigenvalue (a 65x shrink per step, ~9 steps to full precision).
@@ -1398,27 +1415,32 @@ __global__ __launch_bounds__(256) void k_bisect(const double* __restrict__ d, co
     const int lane = threadIdx.x & 63;
     const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (j >= nband) return;   // whole wave; no barrier follows
-    double lo = 1e300, hi = -1e300, emax2 = 0;
+    double lo = 1e300, hi = -1e300, emax2 = 0, emin2 = 1e300;
     for (int i = lane; i < n; i += 64) {
         const double r = (i > 0 ? fabs(e[i - 1]) : 0.0) + (i < n - 1 ? fabs(e[i]) : 0.0);
         lo = fmin(lo, de[i].x - r);
         hi = fmax(hi, de[i].x + r);
         emax2 = fmax(emax2, -de[i].y);
+        if (i > 0) emin2 = fmin(emin2, -de[i].y);
     }
     for (int o = 32; o > 0; o >>= 1) {
         lo = fmin(lo, __shfl_xor(lo, o, 64));
         hi = fmax(hi, __shfl_xor(hi, o, 64));
         emax2 = fmax(emax2, __shfl_xor(emax2, o, 64));
+        emin2 = fmin(emin2, __shfl_xor(emin2, o, 64));
     }
     const double pivmin = DBL_MIN * fmax(1.0, emax2);
     const double tnorm = fmax(fabs(lo), fabs(hi));
     lo -= 2.0 * DBL_EPSILON * tnorm * n + 2 * pivmin;
     hi += 2.0 * DBL_EPSILON * tnorm * n + 2 * pivmin;
+    // an |e| below 2^-60 of T's bound: four such steps at exact zeros, as many as lie between two
+    // rescalings, shrink p by 2^-480 at most
+    const bool split = sqrt(emin2) <= 0x1p-60 * tnorm;
     // invariant: sturm(lo) <= j < sturm(hi)
     for (int it = 0; it < 64; ++it) {
         if (hi - lo <= 2.0 * DBL_EPSILON * fmax(fabs(lo), fabs(hi)) + pivmin) break;
         const double x = lo + (hi - lo) * (double)(lane + 1) / 65.0;
-        const int c = sturm(de, n, x);
+        const int c = split ? sturm_split(de, n, x, pivmin) : sturm(de, n, x);
         const unsigned long long above = __ballot(c > j);
         const double x63 = lane_bcast(x, 63);
         if (above == 0ull) {
