@@ -102,12 +102,16 @@ __device__ inline double2 block_sum2(double a, double b, double* red) {
 constexpr unsigned long long RING_EMPTY = 0x7ff4dead5eed0001ull;
 
 // What a reduction needs before it starts, in one launch: a = hcc (both triangles from the
-// lower one), nz words of bar zeroed, and the exchange ring filled with its empty pattern.
+// lower one), nz words of bar zeroed, and the exchange ring filled with its empty pattern.  d is
+// filled with NaN, so that k_bisect reports a reduction that did not write it instead of taking
+// an earlier matrix's.
 __global__ void k_prep(int n, const double2* __restrict__ h, int ldh, double2* __restrict__ a,
-                       unsigned* __restrict__ bar, int nz, double2* __restrict__ ring, size_t nring) {
+                       unsigned* __restrict__ bar, int nz, double* __restrict__ d, double2* __restrict__ ring,
+                       size_t nring) {
     const size_t first = blockIdx.x * (size_t)blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
     const double empty = __longlong_as_double((long long)RING_EMPTY);
     if (first < (size_t)nz) bar[first] = 0u;
+    if (first < (size_t)n) d[first] = empty;
     for (size_t i = first; i < nring; i += stride) ring[i] = make_double2(empty, empty);
     const size_t total = (size_t)n * n;
     for (size_t t = first; t < total; t += stride) {
@@ -2114,7 +2118,7 @@ __global__ __launch_bounds__(1024) void k_chol_inv(int n, const double2* __restr
 // Every set of reductions that can run together then fits: a later one overlaps an earlier one
 // only if it did not wait for it, and then the earlier one was counted.
 namespace {
-constexpr int NXCD = 8;
+constexpr int NXCD = 8, NCU = 256;   // of the whole GPU
 struct SpinEntry {
     hipEvent_t ev;     // completion
     hipStream_t s;
@@ -2182,10 +2186,20 @@ void spin_launch(const void* fn, dim3 grid, dim3 block, void** args, unsigned ld
     L.live.push_back(SpinEntry{ev, s, w, xcd ? at : -1});
 }
 
-bool xcd_available() {
+// Whether the one-XCD forms may run on s.  A stream that is kept to some of the CUs does without
+// them: on the XCD that a launch names, its workgroups might not be resident together.
+bool xcd_available(hipStream_t s) {
     SpinLedger& L = ledger();
-    std::lock_guard<std::mutex> lock(L.m);
-    return L.xcd_ok;
+    {
+        std::lock_guard<std::mutex> lock(L.m);
+        if (!L.xcd_ok) return false;
+    }
+    std::uint32_t mask[NCU / 32] = {};
+    if (hipExtStreamGetCUMask(s, NCU / 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return std::all_of(mask, mask + NCU / 32, [](std::uint32_t m) { return m == ~0u; });
 }
 }  // namespace
 
@@ -2212,26 +2226,28 @@ void eig_probe_xcds(int num_cu) {
     SpinLedger& L = ledger();
     std::lock_guard<std::mutex> lock(L.m);
     if (L.probed) return;
-    L.probed = true;
-    if (num_cu != 256) return;   // 8 XCDs of 32 CUs; a partition of the GPU keeps the device-wide forms
-    constexpr int nb = 256;
-    unsigned ids[nb];
+    if (num_cu != NCU) {
+        L.probed = true;
+        return;   // 8 XCDs of 32 CUs; a partition of the GPU keeps the device-wide forms
+    }
+    unsigned ids[NCU];
     DevBuf<unsigned> dev;
-    dev.reserve(nb);
+    dev.reserve(NCU);
     hipStream_t s;
     APW_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-    hipLaunchKernelGGL(k_xcc_ids, dim3(nb), dim3(64), 0, s, dev.get());
+    hipLaunchKernelGGL(k_xcc_ids, dim3(NCU), dim3(64), 0, s, dev.get());
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(ids, dev.get(), sizeof(ids), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     (void)hipStreamDestroy(s);
     APW_HIP(e);
     bool ok = true;
-    for (int b = 0; b < nb; ++b) ok = ok && ids[b] == ids[b % NXCD];
+    for (int b = 0; b < NCU; ++b) ok = ok && ids[b] == ids[b % NXCD];
     for (int x = 0; x < NXCD; ++x)
         for (int z = 0; z < x; ++z) ok = ok && ids[x] != ids[z];
     std::copy(ids, ids + NXCD, L.xcc);
     L.xcd_ok = ok;
+    L.probed = true;
 }
 
 // sizes of the blocked back-transform's work arrays (doubles) for n x mc
@@ -2364,7 +2380,7 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
     // them; a larger matrix starts on the whole device and its last XCD_MAX columns are reduced on
     // one XCD (kstop: the first of them).  n = 512: 2.32 ms on the whole device, 1.53 ms on one
     // XCD; n = 640: 3.23 ms, 2.27 ms with the last 512 columns there (2.36 with 384, 2.52 with 256)
-    const bool xcd = n > ws.single_max && xcd_available();
+    const bool xcd = n > ws.single_max && xcd_available(s);
     int kstop = xcd && n > XCD_MAX ? n - XCD_MAX : 0;
     const bool only_xcd = xcd && kstop == 0;
     const int ns = n - kstop;   // columns of the one-XCD part
@@ -2376,7 +2392,8 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
     double2* sub = reinterpret_cast<double2*>(ws.sub.get());
     const size_t prep_n = std::max((size_t)n * n, nring);
     hipLaunchKernelGGL(k_prep, dim3((unsigned)std::min<size_t>(2048, (prep_n + 255) / 256)), dim3(256), 0, s, n,
-                       reinterpret_cast<const double2*>(hcc), ldh, A, ws.bar.get(), BAR_WORDS, ring, nring);
+                       reinterpret_cast<const double2*>(hcc), ldh, A, ws.bar.get(), BAR_WORDS, ws.d.get(), ring,
+                       nring);
     APW_LAUNCH_CHECK();
     if (n > 1) {
         // bar[1]: abort word of the exchange polls; V: n x n reflectors
@@ -2391,7 +2408,8 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
         // a tuner's trial starts from an empty ring, and leaves one and a clear abort word
         auto refill = [&] {
             hipLaunchKernelGGL(k_prep, dim3((unsigned)std::min<size_t>(2048, (prep_n + 255) / 256)), dim3(256), 0, s, n,
-                               reinterpret_cast<const double2*>(hcc), ldh, A, ws.bar.get(), BAR_WORDS, ring, nring);
+                               reinterpret_cast<const double2*>(hcc), ldh, A, ws.bar.get(), BAR_WORDS, ws.d.get(), ring,
+                       nring);
             APW_LAUNCH_CHECK();
         };
         // algorithmic HBM bytes: the matrix read once (16 n^2) and the reflectors written
@@ -2610,7 +2628,7 @@ void heevx_vectors(hipStream_t s, EigWorkspace& ws, GemmWorkspace& gws, int num_
 
 const char* eig_fault_text(unsigned word) {
     if (word & 1u) return "subspace eigensolver: an exchange poll of the tridiagonal reduction timed out";
-    if (word & 2u) return "subspace eigensolver: the tridiagonal reduction produced a non-finite value";
+    if (word & 2u) return "subspace eigensolver: the tridiagonal reduction produced a non-finite value or did not run";
     return "subspace eigensolver: no fault";
 }
 

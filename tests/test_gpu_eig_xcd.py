@@ -100,3 +100,21 @@ def test_contexts_come_and_go(torch):
         assert np.array_equal(e, want[0]) and np.array_equal(V, want[1])
         assert np.array_equal(_solve(torch, keep, H, 10)[0], want[0])
     keep.close()
+
+
+@pytest.mark.parametrize("n", [48, 130])
+def test_stream_kept_to_half_of_the_cus(torch, n):
+    """On a caller's stream with a CU mask the workgroups of one XCD need not be resident together:
+    such a context takes the device-wide reduction (12 and 32 workgroups here)."""
+    import ctypes as C
+    from apw import pw
+    torch.zeros(1, device="cuda")
+    hip = C.CDLL("libamdhip64.so")
+    stream = C.c_void_p()
+    mask = (C.c_uint32 * 8)(*([0xffffffff] * 4 + [0] * 4))
+    assert hip.hipExtStreamCreateWithCUMask(C.byref(stream), 8, mask) == 0
+    H = _hermitian(n, n)
+    ctx = pw.Context(0, stream=stream.value)
+    _check(H, *_solve(torch, ctx, H, n // 4))
+    ctx.close()
+    assert hip.hipStreamDestroy(stream) == 0
