@@ -262,7 +262,8 @@ void heevx_vectors(hipStream_t s, EigWorkspace& ws, GemmWorkspace& gws, int num_
 // Looks once per device whether workgroups go to its XCDs in turn, which the one-XCD reductions
 // rely on (call with that device current; without it they are not used).
 void eig_probe_xcds(int num_cu);
-// Forgets the finished reductions of a stream that is about to be destroyed (synchronised).
+// Forgets the finished reductions of a stream whose context ends (synchronised; it may be destroyed
+// next, or another context may still use it).
 void eig_forget_stream(hipStream_t s);
 // Sizes ws for every n <= nmax, so heevx_lowest allocates nothing (a growing workspace
 // frees and allocates, and hipFree waits for the device).

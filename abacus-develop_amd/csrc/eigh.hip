@@ -21,11 +21,11 @@
 #include <cfloat>
 #include <cmath>
 #include <cstdlib>
-#include <deque>
 #include <mutex>
 #include <vector>
 
 #include "apw_internal.hpp"
+#include "spin_ledger.hpp"
 
 namespace apw {
 namespace {
@@ -2107,34 +2107,31 @@ __global__ __launch_bounds__(1024) void k_chol_inv(int n, const double2* __restr
 
 }  // namespace
 
-// Launches of the multi-workgroup reductions, whose workgroups wait on each other's ring values,
-// may run at the same time on several streams only while all their workgroups fit on the GPU
-// together (each workgroup fits one CU): then none can wait on a workgroup that cannot start, and
-// ordinary kernels beside them always finish and free their CUs.  A device-wide ledger keeps the
-// reductions not known to have finished, in launch order, with the CUs they need on each XCD: a
-// device-wide form an eighth of its workgroups on every XCD, a one-XCD form all of its workgroups
-// on one, the least loaded.  A new one that would not fit first makes its stream wait for the
-// oldest of the other streams' (its own stream's are over before it starts), as many as needed.
-// Every set of reductions that can run together then fits: a later one overlaps an earlier one
-// only if it did not wait for it, and then the earlier one was counted.
 namespace {
-constexpr int NXCD = 8, NCU = 256;   // of the whole GPU
-struct SpinEntry {
-    hipEvent_t ev;     // completion
-    hipStream_t s;
-    int w, xcd;        // workgroups; the XCD they run on, or -1: all
+constexpr int NCU = 256;   // of the whole GPU
+struct HipSpinApi {
+    using Stream = hipStream_t;
+    using Event = hipEvent_t;
+    static bool finished(hipEvent_t ev) { return hipEventQuery(ev) == hipSuccess; }
+    static bool running(hipEvent_t ev) { return hipEventQuery(ev) == hipErrorNotReady; }
+    static void wait(hipStream_t s, hipEvent_t ev) { APW_HIP(hipStreamWaitEvent(s, ev, 0)); }
+    static hipEvent_t create() {
+        hipEvent_t ev;
+        APW_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+        return ev;
+    }
+    static void record(hipEvent_t ev, hipStream_t s) { APW_HIP(hipEventRecord(ev, s)); }
+    static void destroy(hipEvent_t ev) { (void)hipEventDestroy(ev); }
 };
-struct SpinLedger {
-    std::mutex m;
-    std::deque<SpinEntry> live;
-    std::vector<SpinEntry> pool;   // finished
+constexpr int NXCD = SpinLedger<HipSpinApi>::NXCD;
+struct DeviceLedger : SpinLedger<HipSpinApi> {
     // one-XCD forms: the XCC ids in the order in which workgroups go to them, once probed
     bool probed = false, xcd_ok = false;
     unsigned xcc[NXCD] = {};
 };
-SpinLedger g_ledger[64];
+DeviceLedger g_ledger[64];
 
-SpinLedger& ledger() {
+DeviceLedger& ledger() {
     int dev = 0;
     APW_HIP(hipGetDevice(&dev));
     return g_ledger[dev & 63];
@@ -2143,53 +2140,20 @@ SpinLedger& ledger() {
 // xcd: choose an XCD and pass its XCC id in *xcc (an argument of the kernel).
 void spin_launch(const void* fn, dim3 grid, dim3 block, void** args, unsigned lds, hipStream_t s, int num_cu,
                  bool xcd = false, unsigned* xcc = nullptr) {
-    SpinLedger& L = ledger();
+    DeviceLedger& L = ledger();
     std::lock_guard<std::mutex> lock(L.m);
     const int w = xcd ? (int)grid.x / NXCD : (int)grid.x;
     APW_CHECK(w <= (xcd ? num_cu / NXCD : num_cu), "tridiagonal reduction: %d workgroups on %d CUs", w, num_cu);
-    while (!L.live.empty() && hipEventQuery(L.live.front().ev) == hipSuccess) {
-        L.pool.push_back(L.live.front());
-        L.live.pop_front();
-    }
-    // load[x]: eighths of CUs, a device-wide width rounded up to the same share of every XCD
-    int load[NXCD] = {};
-    auto add = [&](const SpinEntry& g, int sign) {
-        for (int x = 0; x < NXCD; ++x)
-            if (g.xcd < 0 || g.xcd == x) load[x] += sign * (g.xcd < 0 ? (g.w + NXCD - 1) / NXCD * NXCD : NXCD * g.w);
-    };
-    for (const auto& g : L.live)
-        if (g.s != s) add(g, 1);
-    auto place = [&]() {   // the XCD to run on (0 for a device-wide form), -1 if it does not fit yet
-        if (xcd) {
-            const int x = (int)(std::min_element(load, load + NXCD) - load);
-            return load[x] + NXCD * w <= num_cu ? x : -1;
-        }
-        return *std::max_element(load, load + NXCD) + (w + NXCD - 1) / NXCD * NXCD <= num_cu ? 0 : -1;
-    };
-    int at = place();
-    for (auto it = L.live.begin(); at < 0 && it != L.live.end(); ++it) {
-        if (it->s == s) continue;
-        APW_HIP(hipStreamWaitEvent(s, it->ev, 0));
-        add(*it, -1);
-        at = place();
-    }
-    if (xcd) *xcc = L.xcc[at];
-    APW_HIP(hipLaunchKernel(fn, grid, block, args, lds, s));
-    hipEvent_t ev;
-    if (!L.pool.empty()) {
-        ev = L.pool.back().ev;
-        L.pool.pop_back();
-    } else {
-        APW_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    }
-    APW_HIP(hipEventRecord(ev, s));
-    L.live.push_back(SpinEntry{ev, s, w, xcd ? at : -1});
+    L.launch(s, w, xcd, num_cu, [&](int at) {
+        if (xcd) *xcc = L.xcc[at];
+        APW_HIP(hipLaunchKernel(fn, grid, block, args, lds, s));
+    });
 }
 
 // Whether the one-XCD forms may run on s.  A stream that is kept to some of the CUs does without
 // them: on the XCD that a launch names, its workgroups might not be resident together.
 bool xcd_available(hipStream_t s) {
-    SpinLedger& L = ledger();
+    DeviceLedger& L = ledger();
     {
         std::lock_guard<std::mutex> lock(L.m);
         if (!L.xcd_ok) return false;
@@ -2203,27 +2167,14 @@ bool xcd_available(hipStream_t s) {
 }
 }  // namespace
 
-// An event may outlive the stream it was last recorded on, but not be queried then: a query that
-// looked at a freed stream has failed as if that stream were being captured.
 void eig_forget_stream(hipStream_t s) {
-    SpinLedger& L = ledger();
+    DeviceLedger& L = ledger();
     std::lock_guard<std::mutex> lock(L.m);
-    auto drop = [&](auto& list) {
-        for (auto it = list.begin(); it != list.end();) {
-            if (it->s == s) {
-                (void)hipEventDestroy(it->ev);
-                it = list.erase(it);
-            } else {
-                ++it;
-            }
-        }
-    };
-    drop(L.live);
-    drop(L.pool);
+    L.forget(s);
 }
 
 void eig_probe_xcds(int num_cu) {
-    SpinLedger& L = ledger();
+    DeviceLedger& L = ledger();
     std::lock_guard<std::mutex> lock(L.m);
     if (L.probed) return;
     if (num_cu != NCU) {
