@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <deque>
 #include <functional>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -69,17 +70,25 @@ struct DevBuf {
         p = nullptr;
         n = 0;
     }
-    // grow-only; contents are not preserved
-    void reserve(size_t count) {
-        if (count <= n) return;
+    // grow-only; contents are not preserved.  A failure leaves the buffer empty.
+    hipError_t try_reserve(size_t count) {
+        if (count <= n) return hipSuccess;
         release();
-        hipError_t e = hipMalloc(&p, count * sizeof(T) + 256);
-        if (e != hipSuccess) {
+        const hipError_t e = hipMalloc(&p, count * sizeof(T) + 256);
+        if (e == hipSuccess) {
+            n = count;
+        } else {
             p = nullptr;
+            (void)hipGetLastError();   // not for the next launch's check
+        }
+        return e;
+    }
+    void reserve(size_t count) {
+        const hipError_t e = try_reserve(count);
+        if (e != hipSuccess) {
             set_error("hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
             throw Error{APW_ENOMEM};
         }
-        n = count;
     }
     T* get() const { return p; }
 };
@@ -163,6 +172,13 @@ struct EigWorkspace {
     int single_max = 0;
 };
 
+// S and X of the density pass for more bands than a Hamiltonian's own hold, shared by the
+// Hamiltonians of a context: m is held while a call uses them.
+struct RhoWorkspace {
+    std::mutex m;
+    DevBuf<double> S, X;
+};
+
 // work arrays of the generalized (pencil) solver
 struct GenWorkspace {
     DevBuf<double> a, r, t, x, c, t2, y;
@@ -182,6 +198,7 @@ struct apw_ctx {
     apw::GemmWorkspace gws;
     apw::EigWorkspace ews;   // subspace eigensolver workspace of apw_dnevx_op
     apw::GenWorkspace gen;   // and of apw_dngvx_op / apw_dngvd_op
+    apw::RhoWorkspace rho;   // of apw_psi_to_rho
     apw::DevBuf<int> status;
     apw::DevBuf<double> vnl_tau;   // atom positions of apw_getvnl
     apw::DevBuf<double> io_stage;  // bands of a wavefunction file, file order

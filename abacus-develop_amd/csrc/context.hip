@@ -204,7 +204,8 @@ int apw_ctx_fill_workspaces(apw_ctx* ctx, double value) {
         apw::EigWorkspace& e = ctx->ews;
         apw::GenWorkspace& q = ctx->gen;
         for (apw::DevBuf<double>* b : {&ctx->scratch, &ctx->gws.part, &ctx->gws.tune_c, &e.a, &e.v, &e.tau, &e.d, &e.e,
-                                       &e.ring, &e.sub, &e.z, &e.zc, &e.wy, &q.a, &q.r, &q.t, &q.x, &q.c, &q.t2, &q.y}) {
+                                       &e.ring, &e.sub, &e.z, &e.zc, &e.wy, &q.a, &q.r, &q.t, &q.x, &q.c, &q.t2, &q.y,
+                                       &ctx->rho.S, &ctx->rho.X}) {
             if (!b->get()) continue;
             hipLaunchKernelGGL(apw::k_fill, dim3((unsigned)std::min<size_t>(4096, (b->n + 255) / 256)), dim3(256), 0,
                                ctx->stream, b->n, value, b->get());

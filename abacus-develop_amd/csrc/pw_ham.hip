@@ -195,6 +195,8 @@ __global__ void k_cols_addf(int rows, int nb, const float2* __restrict__ in, int
     }
 }
 
+constexpr size_t RHO_BYTES = (size_t)3 << 30;   // S and X of one launch of the density pass
+
 int grid_for(size_t n) { return (int)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 16384)); }
 
 }  // namespace
@@ -601,17 +603,32 @@ int apw_psi_to_rho(apw_ham* ham, const double* psi, int ldpsi, int nbands, const
         for (int b = 0; b < nbands; ++b) w[b] = wg[b] / omega;
         h.wts.reserve(nbands);
         APW_HIP(hipMemcpyAsync(h.wts.get(), w.data(), nbands * sizeof(double), hipMemcpyHostToDevice, s));
-        // bands per launch: sixteen of H|psi>'s chunks (3 GB of S + X).  Each launch of the x pass
-        // reads and writes rho once, which costs more than the intermediates leaving the
-        // Infinity Cache (432 bands of 160^3: 4 bands a launch 9.46 ms, 16 8.77, 32 8.18, 64 7.72,
-        // 108 7.52)
-        const int rc = std::min(nbands, 16 * h.chunk);
+        // Bands per launch: each launch of the x pass reads and writes rho once, which costs more
+        // than the intermediates leaving the Infinity Cache (432 bands of 160^3: 4 bands a launch
+        // 9.46 ms, 16 8.77, 32 8.18, 64 7.72, 108 7.52).  So as many as RHO_BYTES of S and X hold,
+        // in the context's workspace; fewer where the memory is not there, and from H|psi>'s chunk
+        // down in the Hamiltonian's own.
+        int rc = std::min(nbands, h.chunk);
+        double *S = h.S.get(), *X = h.X.get();
+        apw::RhoWorkspace& ws = h.ctx->rho;
+        std::unique_lock<std::mutex> lock(ws.m, std::defer_lock);
+        for (int n = (int)std::min<size_t>({apw::RHO_BYTES / (h.grid.bytes_S(16) + h.grid.bytes_X(16)), 4096, (size_t)nbands});
+             n > rc; n /= 2) {
+            if (!lock.owns_lock()) lock.lock();
+            if (ws.S.try_reserve(2 * h.grid.bytes_S(1) * n) == hipSuccess &&
+                ws.X.try_reserve(2 * h.grid.bytes_X(1) * n) == hipSuccess) {
+                rc = n;
+                S = ws.S.get();
+                X = ws.X.get();
+                break;
+            }
+            ws.S.release();
+            ws.X.release();
+        }
         for (int b0 = 0; b0 < nbands; b0 += rc) {
             const int n = std::min(rc, nbands - b0);
-            h.S.reserve(2 * h.grid.bytes_S(1) * n);
-            h.X.reserve(2 * h.grid.bytes_X(1) * n);
             apw::psi_to_rho(s, h.grid, psi + (size_t)2 * b0 * ldpsi, ldpsi, n, h.wts.get() + b0, rho,
-                            add != 0 || b0 > 0, h.S.get(), h.X.get(), &h.ctx->prof);
+                            add != 0 || b0 > 0, S, X, &h.ctx->prof);
         }
         APW_HIP(hipStreamSynchronize(s));
         return APW_OK;
