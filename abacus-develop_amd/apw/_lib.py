@@ -110,6 +110,7 @@ PROTOTYPES = {
     "apw_tune_save": (_i, [C.c_char_p]),
     "apw_tune_clear": (_i, []),
     "apw_tune_stats": (_i, [C.POINTER(C.c_longlong)] * 4),
+    "apw_tune_refused": (_i, [C.POINTER(C.c_longlong)]),
     "apw_tune_entry": (_i, [_i, C.c_char_p, _i, C.POINTER(_i), C.POINTER(_i), C.POINTER(_d)]),
     "apw_zgemm_noalloc": (_i, [_vp, _ch, _ch, _i, _i, _i, C.POINTER(_d), _vp, _i, _vp, _i, C.POINTER(_d), _vp, _i]),
 }

@@ -596,10 +596,12 @@ def tune_clear():
 
 
 def tune_stats():
-    """{entries, hits, misses, tuned} of the process-wide table."""
-    v = [C.c_longlong() for _ in range(4)]
-    check(_tlib().apw_tune_stats(*[C.byref(x) for x in v]))
-    return dict(zip(("entries", "hits", "misses", "tuned"), (x.value for x in v)))
+    """{entries, hits, misses, tuned, refused} of the process-wide table; refused: the hits whose
+    choice no longer exists, so that the fixed rule ran."""
+    v = [C.c_longlong() for _ in range(5)]
+    check(_tlib().apw_tune_stats(*[C.byref(x) for x in v[:4]]))
+    check(_tlib().apw_tune_refused(C.byref(v[4])))
+    return dict(zip(("entries", "hits", "misses", "tuned", "refused"), (x.value for x in v)))
 
 
 def tune_entries():

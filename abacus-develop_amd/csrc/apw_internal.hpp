@@ -225,7 +225,9 @@ struct DeviceGuard {
 // Process-wide table of measured choices (two ints per key).  tune_mode(): 0 = fixed rules,
 // 1 = the table, fixed rules on a miss, 2 = as 1 and a miss is measured and recorded.
 int tune_mode();
-bool tune_find(const std::string& key, int& a, int& b);
+// The table's choice for key, where there is one and valid(a, b) takes it (a table may hold choices
+// of an earlier version).
+bool tune_find(const std::string& key, int& a, int& b, const std::function<bool(int, int)>& valid);
 void tune_store(const std::string& key, int a, int b, double us);
 // Fastest of reps timed runs of run() on stream s (after one untimed run), in microseconds.
 double time_on_stream(hipStream_t s, int reps, const std::function<void()>& run);

@@ -2431,7 +2431,7 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
                 std::snprintf(key, sizeof(key), "tridiag reg n=%d cu=%d", (n + 31) / 32 * 32, num_cu);
                 int a = 0, b = 0;
                 const int wmax = std::min(num_cu, 256);
-                if (tune_find(key, a, b) && a >= w_min && a <= wmax) {
+                if (tune_find(key, a, b, [&](int c, int) { return c >= w_min && c <= wmax; })) {
                     w = a;
                 } else if (tmode == 2) {
                     std::vector<int> cand;
@@ -2475,7 +2475,7 @@ void heevx_values(hipStream_t s, EigWorkspace& ws, int num_cu, int n, int ldh, c
                 char key[96];
                 std::snprintf(key, sizeof(key), "tridiag rows n=%d cu=%d", (n + 31) / 32 * 32, num_cu);
                 int a = 0, b = 0;
-                if (tune_find(key, a, b) && a >= wmin && a <= wmax && b == 0) {
+                if (tune_find(key, a, b, [&](int c, int z) { return c >= wmin && c <= wmax && z == 0; })) {
                     w = a;
                 } else if (tmode == 2) {
                     std::vector<int> cand;

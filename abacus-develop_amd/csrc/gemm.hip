@@ -574,7 +574,7 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
         std::snprintf(key, sizeof(key), "gemm %s %c%c m=%d n=%d k=%d cu=%d", prec_tag, "NTC"[oa], "NTC"[ob],
                       bucket(m), bucket(n), bucket(k), cus);
         int a = 0, b = 0;
-        if (tune_find(key, a, b) && has(a) && b >= 0 && b <= 6) {
+        if (tune_find(key, a, b, [&](int v, int oc) { return has(v) && oc >= 0 && oc <= 6; })) {
             variant = a;
             occ = b;
         } else if (tmode == 2) {

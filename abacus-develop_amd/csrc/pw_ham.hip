@@ -283,7 +283,7 @@ void Ham::tune_local() {
         std::snprintf(key, sizeof(key), "fft %s %dx%dx%d npw=%d cu=%d", pi ? "f32" : "f64", grid.nx, grid.ny, grid.nz,
                       npw, ctx->num_cu);
         int a = 0, b = 0;
-        if (tune_find(key, a, b) && a >= 1 && a <= 256 && b >= 0 && b <= 7) {
+        if (tune_find(key, a, b, [](int c, int sc) { return c >= 1 && c <= 256 && sc >= 0 && sc <= 7; })) {
             ch = a;
             grid.sched[pi] = b;
             continue;

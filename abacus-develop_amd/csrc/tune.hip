@@ -33,6 +33,7 @@ struct Table {
     int mode = 0;
     std::map<std::string, Entry> entries;
     long long hits = 0, misses = 0, tuned = 0;
+    long long refused = 0;   // hits whose choice no longer exists
 };
 
 Table& table() {
@@ -48,7 +49,7 @@ int tune_mode() {
     return t.mode;
 }
 
-bool tune_find(const std::string& key, int& a, int& b) {
+bool tune_find(const std::string& key, int& a, int& b, const std::function<bool(int, int)>& valid) {
     Table& t = table();
     std::lock_guard<std::mutex> lk(t.mu);
     auto it = t.entries.find(key);
@@ -57,6 +58,10 @@ bool tune_find(const std::string& key, int& a, int& b) {
         return false;
     }
     ++t.hits;
+    if (!valid(it->second.a, it->second.b)) {
+        ++t.refused;
+        return false;
+    }
     a = it->second.a;
     b = it->second.b;
     return true;
@@ -112,7 +117,7 @@ int apw_tune_clear(void) {
     apw::Table& t = apw::table();
     std::lock_guard<std::mutex> lk(t.mu);
     t.entries.clear();
-    t.hits = t.misses = t.tuned = 0;
+    t.hits = t.misses = t.tuned = t.refused = 0;
     return APW_OK;
 }
 
@@ -178,6 +183,16 @@ int apw_tune_stats(long long* entries, long long* hits, long long* misses, long 
         *hits = t.hits;
         *misses = t.misses;
         *tuned = t.tuned;
+        return (int)APW_OK;
+    });
+}
+
+int apw_tune_refused(long long* refused) {
+    return apw::guarded([&] {
+        APW_CHECK(refused, "apw_tune_refused: null argument");
+        apw::Table& t = apw::table();
+        std::lock_guard<std::mutex> lk(t.mu);
+        *refused = t.refused;
         return (int)APW_OK;
     });
 }

@@ -510,7 +510,7 @@ def main():
 
     if tune is not None:
         st = pw.tune_stats()
-        tune.update(hits=st["hits"], misses=st["misses"])
+        tune.update(hits=st["hits"] - st["refused"], misses=st["misses"], refused=st["refused"])
         # the same FP32-mixed solve with the fixed rules (a Hamiltonian built without the table)
         pw.tune_set_mode(pw.TUNE_FIXED)
         ham0 = pw.HamiltPW(ctx, s)

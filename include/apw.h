@@ -376,6 +376,7 @@ int apw_tune_load(const char* path);   /* returns the number of entries read */
 int apw_tune_save(const char* path);   /* returns the number of entries written */
 int apw_tune_clear(void);
 int apw_tune_stats(long long* entries, long long* hits, long long* misses, long long* tuned);
+int apw_tune_refused(long long* refused);   /* hits whose choice no longer exists: not taken */
 int apw_tune_entry(int i, char* key, int key_cap, int* a, int* b, double* us);
 /* dnevx_op<complex<double>, DEVICE_GPU> (dngvd_op.h:85-107): lowest nbands eigenpairs
  * of the Hermitian nstart x nstart matrix hcc (lower triangle, ld ldh).  eigenvalue:

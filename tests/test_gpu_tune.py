@@ -150,3 +150,63 @@ def test_every_gemm_plan(torch, tuner, tmp_path, prec, ta, m, n, k):
             tried += 1
     print(prec, ta, key, tried, "plans")
     ctx.close()
+
+
+# the plans that exist: FP64 and FP32 products have one tile in two orders, the x32 form nine
+PLANS = {"f64": (12, 13), "f32": (12, 13), "x32": (0, 1, 4, 5, 6, 7, 9, 10, 11)}
+
+
+def _force(pw, path, key, choice):
+    import json
+    path.write_text('{"version": 1, "entries": [\n' + json.dumps({"key": key, "choice": choice, "us": 1.0}) + "\n]}\n")
+    pw.tune_clear()
+    assert pw.tune_load(str(path)) == 1
+    pw.tune_set_mode(pw.TUNE_CACHE)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "x32"])
+@pytest.mark.parametrize("ta,m,n,k", [("N", 3001, 70, 100), ("C", 70, 90, 5003), ("C", 130, 150, 700)])
+def test_every_existing_plan_is_taken(torch, tuner, tmp_path, prec, ta, m, n, k):
+    pw = tuner
+    ctx = pw.Context(0)
+    rng = np.random.default_rng(12)
+    rows, cols = (k, m) if ta == "C" else (m, k)
+    dt = torch.complex64 if prec == "f32" else torch.complex128
+
+    def operand(*shape):
+        x = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+        return x.astype(np.complex64).astype(np.complex128) if prec == "f32" else x
+
+    A, B, Cm = operand(cols, rows), operand(n, k), operand(n, m)
+    dA, dB = torch.from_numpy(A).to(dt).cuda(), torch.from_numpy(B).to(dt).cuda()
+    alpha, beta = 0.7 - 0.2j, 0.3 + 0.1j
+    opa = A.T.conj().T if ta == "C" else A.T
+    want = alpha * (opa @ B.T) + beta * Cm.T
+    mag = np.abs(alpha) * (np.abs(opa) @ np.abs(B.T)) + np.abs(beta) * np.abs(Cm.T)
+    eps = 6e-8 if prec in ("f32", "x32") else np.finfo(float).eps
+    bound = 8 * np.sqrt(k) * eps * mag + 1e-13
+
+    def run():
+        out = torch.from_numpy(Cm).to(dt).cuda()
+        pw.gemm_op(ctx, ta, "N", m, n, k, alpha, dA, rows, dB, k, beta, out, m, x32=(prec == "x32"))
+        ctx.synchronize()
+        return out.cpu().numpy().astype(np.complex128).T
+
+    fixed = run()
+    pw.tune_set_mode(pw.TUNE_MEASURE)
+    run()
+    (key, _, _), = pw.tune_entries()
+    for v in PLANS[prec]:
+        for occ in (0, 1, 2, 6):
+            _force(pw, tmp_path / "plan.json", key, [v, occ])
+            got = run()
+            st = pw.tune_stats()
+            assert st["hits"] == 1 and st["refused"] == 0, (prec, v, occ)
+            err = np.abs(got - want)
+            assert (err <= bound).all(), (prec, ta, v, occ, (err / bound).max())
+    # a plan of an earlier version: found, refused, and the fixed rule runs
+    _force(pw, tmp_path / "plan.json", key, [3, 0])
+    assert np.array_equal(run(), fixed)
+    st = pw.tune_stats()
+    assert st["hits"] == 1 and st["refused"] == 1
+    ctx.close()
