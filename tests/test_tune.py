@@ -57,3 +57,20 @@ def test_committed_cache_loads():
     keys = [k for k, _, _ in pw.tune_entries()]
     assert any(k.startswith("gemm ") for k in keys) and any(k.startswith("fft ") for k in keys)
     pw.tune_clear()
+
+
+def test_committed_cache_names_choices_that_exist():
+    """On the GPU that the table was measured on (256 CUs) every entry can be looked up and taken."""
+    import json
+    from apw import pw
+    plans = {"f64": (12, 13), "f32": (12, 13), "x32": (0, 1, 4, 5, 6, 7, 9, 10, 11)}
+    for e in json.load(open(pw.TUNE_CACHE_FILE))["entries"]:
+        words, (a, b) = e["key"].split(), e["choice"]
+        if words[0] == "gemm":
+            assert a in plans[words[1]] and 0 <= b <= 6, e
+        elif words[0] == "fft":
+            assert 1 <= a <= 256 and 0 <= b <= 7, e
+        else:   # columns in LDS up to 704, split by rows above; at least n / 8 workgroups there
+            assert words[0] == "tridiag", e
+            n = int(words[2][2:])
+            assert (512 < n <= 704 if words[1] == "reg" else 704 < n <= 2016 and a >= n // 8) and a <= 256, e
