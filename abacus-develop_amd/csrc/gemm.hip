@@ -440,7 +440,7 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     // of 16 (half the barriers); 10: 64 x 64 with a k step of 16 and 11: the same XCD-aware
     // (split-K candidates: each staged column of a k-contiguous operand is 256 bytes, not 128).
     // occ > 0 splits k so that every workgroup of the launch is resident at once (occ
-    // workgroups per CU: floor of the resident slots over the tiles, at least 64 of k per
+    // workgroups per CU: floor of the resident slots over the tiles, at least 64 or 32 of k per
     // split; a launch with a partial last round of workgroups ran up to 1.5x longer); occ = 0
     // does not split.
     static const int VBM[14] = {64, 64, 0, 0, 128, 64, 64, 64, 0, 128, 64, 64, ZP_BM, ZP_BM};
@@ -460,7 +460,13 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
             };
             while (sp > 1 && (long)share() * 8 > slots) --sp;
         }
-        sp = std::max(1, std::min(std::min(sp, std::max(1, k / 64)), 256));
+        // of k a split takes 64 at least, FP64 and FP32 products 32 while that leaves one workgroup
+        // a CU: the few steps of a small product's k are its time (c128, old 64 x 32 tiles, 64 and
+        // 32 of k: 96 x 96 x 700 13.4, 16.3 and 13.3 us; c64 11.5, 13.8 and 11.9), while with
+        // more workgroups the partial products are (300 x 300 x 700 23.1, 20.0 and 23.4)
+        int most = k / 64;
+        if (!X32) most = std::max(most, std::min(k / 32, (int)(cus / tiles)));
+        sp = std::max(1, std::min({sp, most, 256}));
         int kc = (k + sp - 1) / sp;
         kc = (kc + BKMAX - 1) / BKMAX * BKMAX;
         return (k + kc - 1) / kc;

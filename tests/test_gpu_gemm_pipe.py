@@ -135,3 +135,11 @@ def test_same_bits(torch, tuner, m, n, k, single):
     eps = np.finfo(np.float32 if single else np.float64).eps
     assert np.abs(got - want).max() <= 8 * eps * np.sqrt(k) * 2 * np.sqrt(k)
     assert all(torch.equal(o, outs[0]) for o in outs[1:])
+
+
+# splits of 32 to 63 of k: up to one workgroup a CU (256), the last split short
+@pytest.mark.parametrize("ops", ["CN", "NN", "TC"])
+@pytest.mark.parametrize("m,n,k", [(5, 3, 128), (96, 96, 700), (130, 33, 161), (512, 96, 1031), (1000, 1000, 255)])
+@pytest.mark.parametrize("single", [False, True])
+def test_short_splits(torch, tuner, ops, m, n, k, single):
+    _check(torch, tuner, ops, m, n, k, pad=1, single=single)
