@@ -439,10 +439,9 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     // tiles of one k split share one XCD's L2); 9: 128 x 32 with whole m-tiles per XCD and a k step
     // of 16 (half the barriers); 10: 64 x 64 with a k step of 16 and 11: the same XCD-aware
     // (split-K candidates: each staged column of a k-contiguous operand is 256 bytes, not 128).
-    // occ > 0 splits k so that every workgroup of the launch is resident at once (occ
-    // workgroups per CU: floor of the resident slots over the tiles, at least 64 or 32 of k per
-    // split; a launch with a partial last round of workgroups ran up to 1.5x longer); occ = 0
-    // does not split.
+    // occ > 0 splits k for occ workgroups a CU (floor of these slots over the tiles, at least 64 or
+    // 32 of k per split): every workgroup of the launch is resident at once, or for the c64 rule
+    // below in two full rounds (a partial last round ran up to 1.5x longer); occ = 0 does not split.
     static const int VBM[14] = {64, 64, 0, 0, 128, 64, 64, 64, 0, 128, 64, 64, ZP_BM, ZP_BM};
     static const int VBN[14] = {64, 32, 0, 0, 32, 128, 64, 32, 0, 32, 64, 64, ZP_BN, ZP_BN};
     static const int VOCC[14] = {3, 6, 0, 0, 3, 2, 3, 6, 0, 1, 2, 2, ZP_OCC, ZP_OCC};   // resident workgroups per CU
@@ -477,11 +476,16 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     // else whole m-tiles per XCD where enough n-tiles share the rows of A (c128 three, c64
     // four: 228487 x 256 x 1024 5.33 ms, m-major 5.94; c64 2.80 and 3.18), m-major below that,
     // where the narrow last n-tiles then come last and even out the end (51627 x 97 x 480: 293 us,
-    // per XCD 320; c64 51627 x 160 x 512: 219 and 237).  c64 products of few columns are
-    // split twice as often: the sums of a split are FP32.
+    // per XCD 320; c64 51627 x 160 x 512: 219 and 237).
+    // c64 inner products whose one or two n-tiles end on one at most half full (n <= 32, 65..96) take
+    // twice the splits, two rounds of workgroups with half as long FP32 sums.  512 x n x 51627,
+    // us and relative error with 3 and 6 slots a CU: n = 80 146 (8.4e-7) and 136 (6.0e-7), the
+    // second round evens out full and half-full tiles; n = 24 59 (6.0e-7) and 63 (4.4e-7), taken
+    // for the error, which single precision is short of.  The others pay more for it or gain
+    // nothing: n = 64 106 and 116, n = 40 83 and 89, n = 112 179 both, n = 160 236 and 241.
     // x32: inner products with 64 x 32 tiles when they cover n with fewer columns than 64 x 64
-    // ones (n <= 32, 65..96), else 64 x 64; tall updates 128 x 32 in the XCD-aware order; wide
-    // 64 x 128; else 64 x 64.
+    // ones (again n <= 32, 65..96), else 64 x 64; tall updates 128 x 32 in the XCD-aware order;
+    // wide 64 x 128; else 64 x 64.
     const bool few = n <= 32 || (n > 64 && n <= 96);
     int variant, occ = 0;
     if (!X32) variant = !inner && tall && n > (sizeof(S) == 8 ? 2 : 3) * ZP_BN ? 13 : 12;

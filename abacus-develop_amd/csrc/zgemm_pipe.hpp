@@ -247,9 +247,9 @@ __device__ __forceinline__ void zp_tile(int M, int N, const typename ZpType<R>::
 // XCD L % 8, so each XCD takes whole m-tiles and walks their n-tiles back to back, and the
 // rows of A that they share stay in its L2; a last, narrower n-tile comes after all of those, so
 // that the launch ends on short workgroups (51627 x 160 x 512: 453 -> 437 us, 228487 x 200 x 1024
-// 5.31 -> 4.74 ms, in turn with the others before).  map 2 (k split so that all workgroups are resident,
-// 1-D grid of 8 (zp_share(wide) + zp_share(narrow))): each XCD takes an eighth of the splits, all
-// full-width tiles before those of the last, narrower n-tile, so that the workgroups that meet
+// 5.31 -> 4.74 ms, in turn with the others before).  map 2 (k split for one or two full rounds of
+// workgroups, 1-D grid of 8 (zp_share(wide) + zp_share(narrow))): each XCD takes an eighth of the
+// splits, all full-width tiles before those of the last, narrower n-tile, so that the workgroups that meet
 // on a CU (one every num_cu / 8 of an XCD) are a like mix of both on every CU; with m-major order
 // some CUs got the wide ones only.
 __host__ __device__ inline int zp_share(int tiles) { return (tiles + 7) / 8; }
