@@ -474,9 +474,11 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     const bool inner = tiles_of(64, 64) < 2 * cus && k / 64 > 1;
     // Fixed rule (measured on the Davidson shapes): split over k when the tiles leave CUs idle;
     // else whole m-tiles per XCD where enough n-tiles share the rows of A (c128 three, c64
-    // four: 228487 x 256 x 1024 5.33 ms, m-major 5.94; c64 2.80 and 3.18), m-major below that,
-    // where the narrow last n-tiles then come last and even out the end (51627 x 97 x 480: 293 us,
-    // per XCD 320; c64 51627 x 160 x 512: 219 and 237).
+    // four: 228487 x 256 x 1024 5.40 ms, m-major 6.20; c64 2.78 and 3.19), m-major below that,
+    // where it makes no difference or little (51627 x 97 x 480 290 us both; c64 51627 x 160 x 512
+    // 214 both, 228487 x 128 x 480 690 and 725).  c64 products of one or two k steps are
+    // bound by their stores and have no reads of A worth sharing: m-major (228487 x 256 x 24 207 us,
+    // per XCD 272, the 128 x 32 tiles before 247; at k = 64 and 480 columns 603, 577 and 592).
     // c64 inner products whose one or two n-tiles end on one at most half full (n <= 32, 65..96) take
     // twice the splits, two rounds of workgroups with half as long FP32 sums.  512 x n x 51627,
     // us and relative error with 3 and 6 slots a CU: n = 80 146 (8.4e-7) and 136 (6.0e-7), the
@@ -488,7 +490,8 @@ void gemm_impl(hipStream_t s, GemmWorkspace& ws, int num_cu, char ta, char tb, i
     // wide 64 x 128; else 64 x 64.
     const bool few = n <= 32 || (n > 64 && n <= 96);
     int variant, occ = 0;
-    if (!X32) variant = !inner && tall && n > (sizeof(S) == 8 ? 2 : 3) * ZP_BN ? 13 : 12;
+    const bool shared = sizeof(S) == 8 ? n > 2 * ZP_BN : n > 3 * ZP_BN && k > 2 * ZpType<float>::BK;
+    if (!X32) variant = !inner && tall && shared ? 13 : 12;
     else if (inner) variant = few ? 1 : 0;
     else if (tall) variant = 4;
     else variant = wide ? 5 : 0;

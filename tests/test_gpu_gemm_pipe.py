@@ -143,3 +143,10 @@ def test_same_bits(torch, tuner, m, n, k, single):
 @pytest.mark.parametrize("single", [False, True])
 def test_short_splits(torch, tuner, ops, m, n, k, single):
     _check(torch, tuner, ops, m, n, k, pad=1, single=single)
+
+
+# tall products on either side of the line between the two orders of tiles
+@pytest.mark.parametrize("m,n,k", [(33000, 193, 32), (33000, 193, 33), (33000, 129, 24), (33000, 128, 24)])
+@pytest.mark.parametrize("single", [False, True])
+def test_orders_of_tall_products(torch, tuner, m, n, k, single):
+    _check(torch, tuner, "NN", m, n, k, pad=1, single=single)
