@@ -395,10 +395,10 @@ void launch_pipe(ProfScope& ps, hipStream_t s, int map, int splits, int M, int N
                  int lda, const R* B, int ldb, R* C, int ldc, double ar, double ai, double br, double bi, R* part) {
     using c_t = typename ZpType<R>::c_t;
     const int tm = (M + ZP_BM - 1) / ZP_BM, tn = (N + ZP_BN - 1) / ZP_BN;
-    // the balanced order of map 2 up to four n-tiles (us a product with its reduction, map 0 -> 2:
-    // 640 x 160 x 51627 615 -> 542, 577 x 97 424 -> 404, 160 x 160 199 -> 176, 1024 x 256 x 228487
-    // 5540 -> 5405); with eight the narrow one matters little and m-major shares more of A
-    // (480 x 480 x 228487: 5676, map 2 5811)
+    // the balanced order of map 2 up to four n-tiles (us of device time with the reduction, map 0
+    // and 2: 640 x 160 x 51627 598 and 530, 577 x 97 395 and 369, 160 x 160 184 and 160; without a
+    // narrow tile the same: 1024 x 256 x 228487 5614 and 5609); with eight the narrow one matters
+    // little and m-major shares more of A (a call of 480 x 480 x 228487: 5676, map 2 5811)
     if (map == 0 && splits > 1 && N <= 4 * ZP_BN) map = 2;
     if (map == 0 && tn > 65535) map = 1;   // past the grid's second dimension
     const int narrow = N % ZP_BN ? splits * tm : 0, wide = splits * tm * (N / ZP_BN);

@@ -12,12 +12,13 @@
 //
 // Measured on one MI355X against staging through registers with a prefetch of one step (the
 // loads then had half a step to arrive and both waves of a SIMD waited for them; matrix cores
-// 67 % busy), us a product: c128 CN 1024 x 256 x 228487 6542 -> 5376 (89 TFLOP/s of 8 m n k; the
-// three-product loop alone, from LDS, reaches 98), CN 512 x 160 x 51627 592 -> 427,
-// CN 577 x 97 x 51627 487 -> 397, NN 228487 x 256 x 1024 6607 -> 5333; c64 CN 512 x 160 x 51627
-// 339 -> 229, NN 51627 x 160 x 512 303 -> 219 (155 TFLOP/s).  Waves 2 x 2 instead of stacked: 5997
-// on the first; four stages (two workgroups a CU): 6159; 128 x 32: 6157; 128 x 64 (one
-// workgroup a CU): 7058; 64 x 32: 6070.
+// 67 % busy), us of device time a product with its split-K reduction, after a warm-up (the first
+// ten passes run at lower clocks and take up to 20 % longer): c128 CN 1024 x 256 x 228487 6570 ->
+// 5480 (87 TFLOP/s of 8 m n k; the three-product loop alone, from LDS, reaches 98), CN 512 x 160 x
+// 51627 579 -> 413, CN 577 x 97 x 51627 498 -> 369, NN 228487 x 256 x 1024 6617 -> 5328; c64 CN 512 x
+// 160 x 51627 323 -> 209, NN 51627 x 160 x 512 279 -> 216 (157 TFLOP/s).  The first of these in a
+// program of its own, where this form took 5376: waves 2 x 2 instead of stacked 5997; four stages
+// (two workgroups a CU) 6159; 128 x 32 6157; 128 x 64 (one workgroup a CU) 7058; 64 x 32 6070.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -246,8 +247,8 @@ __device__ __forceinline__ void zp_tile(int M, int N, const typename ZpType<R>::
 // splits); map 1 (1-D grid in x padded to a multiple of 8 m-tiles): workgroup L runs on
 // XCD L % 8, so each XCD takes whole m-tiles and walks their n-tiles back to back, and the
 // rows of A that they share stay in its L2; a last, narrower n-tile comes after all of those, so
-// that the launch ends on short workgroups (51627 x 160 x 512: 453 -> 437 us, 228487 x 200 x 1024
-// 5.31 -> 4.74 ms, in turn with the others before).  map 2 (k split for one or two full rounds of
+// that the launch ends on short workgroups (a call of 51627 x 160 x 512: 453 -> 437 us, 228487 x 200 x
+// 1024 5.31 -> 4.74 ms, against the narrow ones in turn with the others).  map 2 (k split for one or two full rounds of
 // workgroups, 1-D grid of 8 (zp_share(wide) + zp_share(narrow))): each XCD takes an eighth of the
 // splits, all full-width tiles before those of the last, narrower n-tile, so that the workgroups that meet
 // on a CU (one every num_cu / 8 of an XCD) are a like mix of both on every CU; with m-major order
