@@ -70,25 +70,17 @@ struct DevBuf {
         p = nullptr;
         n = 0;
     }
-    // grow-only; contents are not preserved.  A failure leaves the buffer empty.
-    hipError_t try_reserve(size_t count) {
-        if (count <= n) return hipSuccess;
-        release();
-        const hipError_t e = hipMalloc(&p, count * sizeof(T) + 256);
-        if (e == hipSuccess) {
-            n = count;
-        } else {
-            p = nullptr;
-            (void)hipGetLastError();   // not for the next launch's check
-        }
-        return e;
-    }
+    // grow-only; contents are not preserved
     void reserve(size_t count) {
-        const hipError_t e = try_reserve(count);
+        if (count <= n) return;
+        release();
+        hipError_t e = hipMalloc(&p, count * sizeof(T) + 256);
         if (e != hipSuccess) {
+            p = nullptr;
             set_error("hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
             throw Error{APW_ENOMEM};
         }
+        n = count;
     }
     T* get() const { return p; }
 };

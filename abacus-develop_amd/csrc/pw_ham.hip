@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "apw_ham.hpp"
+#include "rho_bands.hpp"
 
 namespace apw {
 namespace {
@@ -194,8 +195,6 @@ __global__ void k_cols_addf(int rows, int nb, const float2* __restrict__ in, int
         out[(size_t)c * ldo + r] = o;
     }
 }
-
-constexpr size_t RHO_BYTES = (size_t)3 << 30;   // S and X of one launch of the density pass
 
 int grid_for(size_t n) { return (int)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 16384)); }
 
@@ -606,24 +605,28 @@ int apw_psi_to_rho(apw_ham* ham, const double* psi, int ldpsi, int nbands, const
         // Bands per launch: each launch of the x pass reads and writes rho once, which costs more
         // than the intermediates leaving the Infinity Cache (432 bands of 160^3: 4 bands a launch
         // 9.46 ms, 16 8.77, 32 8.18, 64 7.72, 108 7.52).  So as many as RHO_BYTES of S and X hold,
-        // in the context's workspace; fewer where the memory is not there, and from H|psi>'s chunk
-        // down in the Hamiltonian's own.
-        int rc = std::min(nbands, h.chunk);
+        // in the context's workspace, fewer where little memory is free; up to H|psi>'s chunk the
+        // Hamiltonian's own.
         double *S = h.S.get(), *X = h.X.get();
         apw::RhoWorkspace& ws = h.ctx->rho;
         std::unique_lock<std::mutex> lock(ws.m, std::defer_lock);
-        for (int n = (int)std::min<size_t>({apw::RHO_BYTES / (h.grid.bytes_S(16) + h.grid.bytes_X(16)), 4096, (size_t)nbands});
-             n > rc; n /= 2) {
-            if (!lock.owns_lock()) lock.lock();
-            if (ws.S.try_reserve(2 * h.grid.bytes_S(1) * n) == hipSuccess &&
-                ws.X.try_reserve(2 * h.grid.bytes_X(1) * n) == hipSuccess) {
-                rc = n;
+        const size_t band_S = 2 * h.grid.bytes_S(1), band_X = 2 * h.grid.bytes_X(1);   // doubles
+        const size_t band_bytes = (band_S + band_X) * sizeof(double);
+        int rc = apw::rho_bands(nbands, h.chunk, band_bytes, 0, 2 * apw::RHO_BYTES);
+        if (rc > h.chunk) {
+            lock.lock();
+            const size_t fit = std::min(ws.S.n / band_S, ws.X.n / band_X);   // bands it holds now
+            if (fit < (size_t)rc) {
+                size_t free_bytes = 0, total = 0;
+                APW_HIP(hipMemGetInfo(&free_bytes, &total));
+                rc = apw::rho_bands(nbands, h.chunk, band_bytes, fit * band_bytes, free_bytes);
+            }
+            if (rc > h.chunk) {
+                ws.S.reserve(band_S * rc);
+                ws.X.reserve(band_X * rc);
                 S = ws.S.get();
                 X = ws.X.get();
-                break;
             }
-            ws.S.release();
-            ws.X.release();
         }
         for (int b0 = 0; b0 < nbands; b0 += rc) {
             const int n = std::min(rc, nbands - b0);

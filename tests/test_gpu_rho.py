@@ -99,6 +99,8 @@ def test_workspace_is_the_contexts(torch):
     assert before - torch.cuda.mem_get_info()[0] < 0.5 * GIB
 
 
+@pytest.mark.skip(reason="with a failing allocation in the call, this ended in a segmentation fault inside the runtime "
+                         "once, late in a run of all tests; the cause is not known.  tests/test_rho_bands.py has the rule")
 def test_little_memory(torch):
     """With two gigabytes left the density is formed with fewer bands a launch."""
     from apw import pw
