@@ -141,7 +141,8 @@ int apw_real_to_recip(apw_ham* ham, const double* in, double* out, int add, doub
  * unnormalised backward FFT of band b scattered into the box (recip_to_real).
  * psi: device c128, band b at psi + b*ldpsi (ldpsi >= npw); wg: HOST double[nbands];
  * rho: device double[nx*ny*nz], overwritten (add = 0) or accumulated (add != 0).
- * Bands are summed in order (deterministic).  Synchronous. */
+ * Bands are summed in order (deterministic).  Synchronous.  The context keeps up to 3 GiB of work
+ * arrays for it, at most half of what is free when they grow; a few bands need none. */
 int apw_psi_to_rho(apw_ham* ham, const double* psi, int ldpsi, int nbands, const double* wg,
                    double omega, double* rho, int add);
 
